@@ -1508,13 +1508,13 @@ __global__ __launch_bounds__(kBlock) void k_fwd_z(const PoseSlot* __restrict__ s
 // plane write; all threads of the workgroup call it.  TR_IN_PLANE: the
 // transforms' scratch tr lies inside the plane, so every transform waits
 // until no wavefront reads the plane any more.
-template <int N, int PROWS, bool TR_IN_PLANE = false>
-__device__ __forceinline__ void col_inverse(float2 (&acc)[N / (4 * RegShape<N>::LPW)][RegShape<N>::V], float2* pl,
+template <int N, int PROWS, bool TR_IN_PLANE = false, int NW = 4>
+__device__ __forceinline__ void col_inverse(float2 (&acc)[N / (NW * RegShape<N>::LPW)][RegShape<N>::V], float2* pl,
                                             float2* tr, const float2* twr, int lane, int wave, float2* tb, int wx,
                                             int wy, float invG) {
   using RS = RegShape<N>;
   constexpr int L = RS::L, V = RS::V, LPW = RS::LPW;
-  constexpr int LPP = 4 * LPW;
+  constexpr int LPP = NW * LPW;
   constexpr int NPASS = N / LPP;
   // inverse x transforms of the ky lines: value m = x' = n2 + L*m
   int ln = lane % LPW, n2 = lane / LPW;
@@ -1898,6 +1898,13 @@ __device__ __forceinline__ unsigned swap_neg_f16(unsigned h) {
   return r;
 }
 
+// (x, y) -> (y, -x) on a packed FP16 pair (an exact multiply by 1).
+__device__ __forceinline__ unsigned swap_a_f16(unsigned h) {
+  unsigned r;
+  asm("v_pk_mul_f16 %0, %1, 1.0 op_sel:[1,0] op_sel_hi:[0,0] neg_hi:[1,0]" : "=v"(r) : "v"(h));
+  return r;
+}
+
 // A operands shared by the SW wavefronts of a workgroup that own blocks of the
 // same kx rows (SW = 1: each wavefront builds its own): per 8-entry step,
 // wavefront w builds and splits the A values of entries j = w, w + SW, ...
@@ -2229,6 +2236,406 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     // the split products' scales out with 1/G (powers of two: exact)
     const float sc = PR == kAtomF32 ? invG : invG * __int_as_float(uni(__float_as_int(Ld.aunscale))) * (1.f / kAtomYScale);
     col_inverse<N, N, true>(acc, pl, tr, twr, lane, wave, T2 + ((size_t)s * ZH + kz) * (size_t)(N * N), wx, wy, sc);
+  }
+}
+
+// Value of x on lane J of this lane's row of 16 lanes.
+template <int J>
+__device__ __forceinline__ float row_bcast(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + J, 0xf, 0xf, true));
+}
+template <int J>
+__device__ __forceinline__ unsigned row_bcast(unsigned x) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + J, 0xf, 0xf, true);
+}
+
+// 64-point transform of 32 lines by one wavefront in registers: lane
+// (line, p), p = lane / 32, holds t[i][n1] = x[n2 + 8 n1], n2 = 4 p + i, i < 4.
+// The same arithmetic as reg_fft<64, S> (DFT_8 over n1, twiddles W^(n2 k1),
+// DFT_8 over n2); the transpose between the two is a register swap with the
+// lane of the other p.  Leaves t[i][m] = X[k1 + 8 m], k1 = 4 p + i.
+// twr: the twiddles of n2 = 4 p (8 per n2).
+template <int S>
+__device__ __forceinline__ void pair_fft64(float2 (&t)[4][8], const float2* twr) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    SmallDFT<8, S>::run(t[i]);
+#pragma unroll
+    for (int k1 = 1; k1 < 8; ++k1) {
+      float2 w = twr[i * 8 + k1];
+      if (S > 0) w.y = -w.y;
+      t[i][k1] = c_mul(t[i][k1], w);
+    }
+  }
+  float2 u[4][8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[i][k].x), __float_as_uint(t[i][4 + k].x), false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(t[i][k].y), __float_as_uint(t[i][4 + k].y), false, false);
+      u[k][i] = make_float2(__uint_as_float(x[0]), __uint_as_float(y[0]));
+      u[k][4 + i] = make_float2(__uint_as_float(x[1]), __uint_as_float(y[1]));
+    }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    SmallDFT<8, S>::run(u[k]);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) t[k][m] = u[k][m];
+  }
+}
+
+// LDS of k_mid_atoms_x3: the split y factors of up to ROWS atoms,
+// [ky / 32][part][atom][ky % 32] packed FP16 pairs, then the staged entries.
+// A (ky half, part) region is 8 bytes longer than its rows, so its words are
+// no multiple of 256 bytes and no 255 words apart from the next region's: the
+// compiler then reads each into its operand register directly instead of
+// pairing them into two-register reads with moves after.
+struct AtomTab {
+  static constexpr int NP = 2;  // kz planes per workgroup
+  static constexpr int ROWS = 84;
+  static constexpr int ROW = 32 * 4;
+  static constexpr int REG = ROWS * ROW + 8;
+  static constexpr int ENT = (6 * REG + 15) & ~15;       // byte offset of the staged entries
+  static constexpr int LDS = 80 * 1024 - 1024;           // with the twiddles: two workgroups per CU
+  static constexpr int TAIL = 16;                        // zero entries after the staged ones (read ahead)
+  // padded entries of a ligand of ROWS atoms: vdW and elec lists, each channel to a multiple of 8
+  static constexpr int MAXENT = ROWS + 7 * (kMaxCh - 1) + ROWS + 7 + TAIL;
+  static_assert(ENT + MAXENT * (16 * NP + 8) <= LDS, "table and entries fit");
+};
+
+// The 64-point mid stage of the atom form with exact three-part products
+// (atom_products 2), for ligands of up to AtomTab::ROWS atoms: as k_mid_atoms,
+// bit for bit, by two wavefronts per kz plane, wavefront w owning the 32 kx
+// rows 32 w .. and all 64 ky (two 32 x 32 blocks that share the A operands),
+// at two wavefronts per SIMD and up to 256 registers.  A workgroup takes the
+// planes 2 i and 2 i + 1 of a group of poses.
+//
+// What bounds it: a step of 8 entries is 24 matrix-core instructions (768
+// cycles) beside ~106 vector instructions, and the two overlap only as far as
+// the wavefronts' instruction streams are interleaved.  Four wavefronts per
+// plane at four per SIMD (k_mid_atoms) built every operand twice (141 vector
+// instructions per block and step, most of the splits at half rate), waited
+// on one table lookup after the other, and on each protein load in turn.
+// Here:
+//   - the y factors do not depend on kz, the channel or the kx rows: each
+//     atom's split B operands are built once per (pose, workgroup) into an LDS
+//     table and gathered by the vdW and the elec entries of the atom;
+//   - one A operand serves both ky blocks, and the imaginary sums reuse B with
+//     the A parts swapped, (a0, a1) -> (a1, -a0);
+//   - an entry's weights sit on four lanes of each 16-lane row and reach the
+//     others by row broadcasts, one LDS read per step;
+//   - the next step's A is built between the current step's imaginary
+//     products, its B is read while the protein product runs, and the
+//     protein loads of a channel are issued 8 at a time ahead of its products;
+//   - the inverse transforms hold a 64-point line in two lanes (pair_fft64):
+//     one exchange with the other wavefront and one plane transpose through
+//     LDS, against two plane transposes and two scratch transposes.
+// Measured, the mid stage of 10 000 poses of 40 atoms: 10.4 -> 9.1 ms (2 331
+// poses of 57 atoms: 2.9 -> 2.5 ms).  Larger ligands keep k_mid_atoms: their
+// table leaves no room for the two workgroups per CU that fill the SIMDs
+// (one plane per workgroup, four per CU, measured the same up to the 44 atoms
+// that fit it).
+template <class P>
+__global__ __launch_bounds__(128 * AtomTab::NP) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mid_atoms_x3(
+    const PoseSlot* __restrict__ slots, const LigandDesc* __restrict__ ligs, const int* __restrict__ pad_atoms,
+    const float* __restrict__ wv, const float* __restrict__ wq, const AtomGrid* __restrict__ ag, int astride,
+    const RotMeta* __restrict__ meta, int nslots, int group, const float2* __restrict__ P3, float2* __restrict__ T2,
+    float invG, const float2* __restrict__ twg) {
+  constexpr int N = P::N, ZH = P::ZH;
+  static_assert(N == 64, "one workgroup holds a 64 x 64 plane");
+  using AT = AtomTab;
+  constexpr int NP = AT::NP;
+  __shared__ __align__(16) unsigned char mem[AT::LDS];  // the table and entries, then the plane
+  __shared__ float2 stw[N];                             // W^m
+  __shared__ float2 stwr[64];                           // register FFT twiddles, [n2][k1]
+  static_assert(NP * N * N * (int)sizeof(float2) <= AT::LDS, "the planes share the table's memory");
+  constexpr int ITEMS = (ZH + NP - 1) / NP;
+  int item, sg;
+  if (!xcd_plane_of(blockIdx.x, ITEMS / 8, ITEMS % 8, (nslots + group - 1) / group, item, sg)) return;
+  const int tid = threadIdx.x;
+  for (int t = tid; t < N; t += blockDim.x) {
+    stw[t] = twg[t];
+    stwr[t] = twg[(t >> 3) * (t & 7)];
+  }
+  auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  const int plane = uni(tid >> 7);
+  const int wave = uni((tid >> 6) & 1);        // of the plane's two
+  const int kz = min(NP * item + plane, ZH - 1);
+  const bool live = NP * item + plane < ZH;    // the last workgroup of a group has one plane
+  float2* pl = reinterpret_cast<float2*>(mem) + plane * (N * N);
+  const int lane = tid & 63;
+  const int part = lane >> 5;                  // half of a step's entries: 4 part .. 4 part + 3
+  const int kxA = 32 * wave + (lane & 31);     // this lane's A row
+  const int esel = 4 * part + (lane & 3);      // the entry whose weights this lane holds
+  __syncthreads();
+  // X_a(k) = W^(k ix) (1 - fx (1 - W^k)): per lane, D = 1 - W^k
+  const float2 dx = make_float2(1.f - stw[kxA].x, -stw[kxA].y);
+  const char* stwb = reinterpret_cast<const char*>(stw);
+  const unsigned char* tabl = mem + (lane & 31) * 4;
+  const int s0 = sg * group, s1 = min(nslots, s0 + group);
+  for (int s = s0; s < s1; ++s) {
+    if (!uni(meta[s].valid)) continue;
+    const int lig = uni(slots[s].lig);
+    const LigandDesc& Ld = ligs[lig];
+    const int nch = uni(Ld.nch), natom = uni(Ld.natom);
+    const int ptot = uni(Ld.pad_start[nch]);
+    const int wx = uni(meta[s].win[0]), wy = uni(meta[s].win[1]);
+    const AtomGrid* ags = ag + (size_t)s * astride;
+    const int nent = ptot + AT::TAIL;
+    // (w Z(kz), fx w Z(kz)) per plane, and (8 ix, table row offset)
+    float4* ef = reinterpret_cast<float4*>(mem + AT::ENT) + plane * nent;
+    uint2* ei = reinterpret_cast<uint2*>(mem + AT::ENT + NP * nent * (int)sizeof(float4));
+    __syncthreads();  // the previous pose's planes are done with the memory
+    {
+      int te = tid;
+      asm volatile("" : "+v"(te));  // the addresses below are not worth registers in the main loop
+      const int pad_off = Ld.pad_off, w_off = Ld.w_off, t_elec = Ld.pad_start[nch - 1];
+      for (int k = te & 127; k < nent; k += 128) {
+        const int a = k < ptot ? pad_atoms[pad_off + k] : -1;
+        float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+        uint2 q = make_uint2(0u, 0u);
+        if (a >= 0) {
+          const AtomGrid g = ags[a];
+          // elec channel: the charge; vdW channels: sqrt(eps) (FillLigandGrid.cpp:45, :97)
+          const float wa = (k >= t_elec ? wq[w_off + a] : wv[w_off + a]) * Ld.ascale;
+          const float2 z0 = stw[(kz * g.iz) % N], z1 = stw[(kz * (g.iz + 1)) % N];
+          const float2 zf = c_fma_s(z1, (float)g.fz, c_scale(z0, (float)(1.0 - g.fz)));
+          const float2 wz = make_float2(wa * zf.x, wa * zf.y);
+          const float fx = (float)g.fx;
+          f = make_float4(wz.x, wz.y, fx * wz.x, fx * wz.y);
+          q = make_uint2(8u * (unsigned)g.ix, (unsigned)(a * AT::ROW));
+        }
+        ef[k] = f;
+        if (plane == 0) ei[k] = q;
+      }
+      const int ky = te & 63;
+      const float2 dk = make_float2(1.f - stw[ky].x, -stw[ky].y);
+      for (int a = 2 * plane + wave; a < natom; a += 2 * NP) {
+        const AtomGrid& g = ags[a];
+        // kAtomYScale Y_a(ky) = W^(ky iy) (kAtomYScale (1 - fy D))
+        const float fy = (float)g.fy * kAtomYScale;
+        const float2 ty = *reinterpret_cast<const float2*>(stwb + atom_tw_bytes<N>(ky, 8u * (unsigned)g.iy));
+        const float hx = fmaf(-fy, dk.x, kAtomYScale), hy = -fy * dk.y;
+        const float yx = fmaf(ty.x, hx, -(ty.y * hy)), yy = fmaf(ty.x, hy, ty.y * hx);
+        unsigned h, m, l;
+        split3_f16(yx, yy, h, m, l);
+        unsigned char* row = mem + a * AT::ROW + (ky >> 5) * (3 * AT::REG) + (ky & 31) * 4;
+        *reinterpret_cast<unsigned*>(row) = h;
+        *reinterpret_cast<unsigned*>(row + AT::REG) = m;
+        *reinterpret_cast<unsigned*>(row + 2 * AT::REG) = l;
+      }
+    }
+    __syncthreads();
+
+    unsigned a[3][4], b[2][3][4];  // a step's operands: [hi, mid, lo][entry]; b per ky block
+    float4 f;                      // the next step's entry
+    uint2 q;
+    float2 tx[4];
+    auto load_entry = [&](int k) {
+      f = ef[k + esel];
+      q = ei[k + esel];
+    };
+    auto load_b = [&]() {
+      auto one = [&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const unsigned char* row = tabl + row_bcast<j>(q.y);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < 3; ++i) b[h][i][j] = *reinterpret_cast<const unsigned*>(row + (h * 3 + i) * AT::REG);
+      };
+      one(std::integral_constant<int, 0>{});
+      one(std::integral_constant<int, 1>{});
+      one(std::integral_constant<int, 2>{});
+      one(std::integral_constant<int, 3>{});
+    };
+    auto load_tx = [&]() {
+      tx[0] = *reinterpret_cast<const float2*>(stwb + atom_tw_bytes<N>(kxA, row_bcast<0>(q.x)));
+      tx[1] = *reinterpret_cast<const float2*>(stwb + atom_tw_bytes<N>(kxA, row_bcast<1>(q.x)));
+      tx[2] = *reinterpret_cast<const float2*>(stwb + atom_tw_bytes<N>(kxA, row_bcast<2>(q.x)));
+      tx[3] = *reinterpret_cast<const float2*>(stwb + atom_tw_bytes<N>(kxA, row_bcast<3>(q.x)));
+    };
+    // (a0, a1) = conj(W^(kx ix) g), g = wZ - fx wZ D, k slots (real, imaginary)
+    auto make_a = [&]() {
+      auto one = [&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const float fz = row_bcast<j>(f.z), fw = row_bcast<j>(f.w);
+        const float gx = fmaf(-fz, dx.x, fmaf(fw, dx.y, row_bcast<j>(f.x)));
+        const float gy = fmaf(-fz, dx.y, fmaf(-fw, dx.x, row_bcast<j>(f.y)));
+        const float a0 = fmaf(tx[j].x, gx, -(tx[j].y * gy));
+        const float a1 = fmaf(-tx[j].x, gy, -(tx[j].y * gx));
+        split3_f16(a0, a1, a[0][j], a[1][j], a[2][j]);
+      };
+      one(std::integral_constant<int, 0>{});
+      one(std::integral_constant<int, 1>{});
+      one(std::integral_constant<int, 2>{});
+      one(std::integral_constant<int, 3>{});
+    };
+    float2 E[2][16];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) E[h][r] = make_float2(0.f, 0.f);
+    mfma_acc16 cr[2], ci[2];
+    float4 pv[2][8];  // the channel's protein spectrum on the two blocks
+    // One step: a and b hold its operands, f and q the next step's entry (at
+    // k + 8).  first: the channel's sums start here; last: they end here, the
+    // protein loads are issued and the next b is read by the caller.
+    auto step = [&](int k, auto first, auto last, const float2* pb) {
+      auto op = [](const unsigned (&r)[4]) { return __builtin_bit_cast(mfma_h8, (mfma_u4){r[0], r[1], r[2], r[3]}); };
+      auto run = [&](mfma_acc16 (&acc)[2], const unsigned (&aa)[3][4]) {
+        const mfma_acc16 zero = {};
+        // (i, j) part pairs of the kept partial products, largest first
+        constexpr int ia[6] = {0, 0, 1, 0, 2, 1}, ib[6] = {0, 1, 0, 2, 0, 1};
+#pragma unroll
+        for (int u = 0; u < 6; ++u)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            acc[h] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                op(aa[ia[u]]), op(b[h][ib[u]]), u == 0 && decltype(first)::value ? zero : acc[h], 0, 0, 0);
+      };
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (decltype(last)::value) {
+#pragma unroll
+        for (int q8 = 0; q8 < 8; ++q8) pv[0][q8] = *reinterpret_cast<const float4*>(pb + q8 * 128);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      load_tx();
+      unsigned as[3][4];
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) as[i][j] = swap_a_f16(a[i][j]);
+      run(cr, a);
+      __builtin_amdgcn_sched_barrier(0);
+      make_a();
+      run(ci, as);
+#pragma unroll
+      for (int u = 0; u < 12; ++u) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // one matrix-core instruction,
+        __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);  // six vector ones
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (decltype(last)::value) {
+#pragma unroll
+        for (int q8 = 0; q8 < 8; ++q8) pv[1][q8] = *reinterpret_cast<const float4*>(pb + (8 + q8) * 128);
+      } else {
+        load_b();
+        load_entry(k + 16);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load_entry(0);
+    load_b();
+    load_tx();
+    make_a();
+    load_entry(8);
+    for (int c = 0; c < nch; ++c) {
+      const int p0 = uni(Ld.pad_start[c]), p1 = uni(Ld.pad_start[c + 1]);
+      const float2* pb = P3 + (((size_t)uni(Ld.pmap[c]) * ZH + kz) * 4 + 2 * wave) * (8 * 128) + lane * 2;
+      if (p1 - p0 > 8) {
+        step(p0, std::true_type{}, std::false_type{}, pb);
+        for (int k = p0 + 8; k < p1 - 8; k += 8) step(k, std::false_type{}, std::false_type{}, pb);
+        step(p1 - 8, std::false_type{}, std::true_type{}, pb);
+      } else {
+        step(p0, std::true_type{}, std::true_type{}, pb);
+      }
+      // sum += conj(L_c) P_c
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (h == 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          load_b();
+          load_entry(p1 + 8);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q8 = 0; q8 < 8; ++q8) {
+          const float4 pq = pv[h][q8];  // registers 2q, 2q + 1
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            const int r = 2 * q8 + u;
+            const float px = u ? pq.z : pq.x, py = u ? pq.w : pq.y;
+            E[h][r].x = fmaf(cr[h][r], px, E[h][r].x);
+            E[h][r].x = fmaf(-ci[h][r], py, E[h][r].x);
+            E[h][r].y = fmaf(cr[h][r], py, E[h][r].y);
+            E[h][r].y = fmaf(ci[h][r], px, E[h][r].y);
+          }
+        }
+      }
+    }
+    // the split products' scales out with 1/G (powers of two: exact)
+    const float sc = invG * __int_as_float(uni(__float_as_int(Ld.aunscale))) * (1.f / kAtomYScale);
+    __syncthreads();  // the table's reads are done
+    int le = tid & 63;
+    asm volatile("" : "+v"(le));
+    const int pe = le >> 5;
+    const float2* twr = stwr + pe * 32;
+    // Lane (ky = 32 wave + lane % 32, pe) takes every kx = n2 + 8 n1 of its ky,
+    // n2 = 4 pe + i: its own rows n1 = 4 wave + r / 4 and the other
+    // wavefront's, i = r % 4.
+    float2 t4[4][8];
+    {
+      float2* xo = pl + wave * (16 * 64) + le;
+      const float2* xi = pl + (1 - wave) * (16 * 64) + le;
+      if (wave == 0) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) xo[r * 64] = E[1][r];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) xo[r * 64] = E[0][r];
+      }
+      __syncthreads();
+      if (wave == 0) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          t4[r & 3][r >> 2] = E[0][r];
+          t4[r & 3][4 + (r >> 2)] = xi[r * 64];
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          t4[r & 3][r >> 2] = xi[r * 64];
+          t4[r & 3][4 + (r >> 2)] = E[1][r];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t4[i][j] = c_scale(t4[i][j], sc);
+    }
+    pair_fft64<1>(t4, twr);  // t4[i][m]: x' = 4 pe + i + 8 m
+    __syncthreads();         // the exchange's reads are done
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const ColBases wb = col_line_k<N>(32 * wave + (le & 31), 4 * pe + i);
+#pragma unroll
+      for (int m = 0; m < 8; ++m)
+        if (8 * m < wx) pl[col_at_k<N>(wb, m)] = t4[i][m];
+    }
+    __syncthreads();
+    if (32 * wave < wx) {
+      // lane (x', pe): ky = n2 + 8 n1
+      const int xp = 32 * wave + (le & 31);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const ColBases rb = col_line_x<N>(xp, 4 * pe + i);
+#pragma unroll
+        for (int n1 = 0; n1 < 8; ++n1) t4[i][n1] = pl[col_at_x<N>(rb, n1)];
+      }
+      pair_fft64<1>(t4, twr);  // t4[i][m]: y' = 4 pe + i + 8 m
+      float2* tb = T2 + ((size_t)s * ZH + kz) * (size_t)(N * N) + xp * 8 + 4 * pe;
+      if (xp < wx && live) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+          if (8 * m < wy) {
+            float4* d = reinterpret_cast<float4*>(tb + m * (N * 8));
+            d[0] = make_float4(t4[0][m].x, t4[0][m].y, t4[1][m].x, t4[1][m].y);
+            d[1] = make_float4(t4[2][m].x, t4[2][m].y, t4[3][m].x, t4[3][m].y);
+          }
+      }
+    }
   }
 }
 
@@ -2867,12 +3274,21 @@ hipError_t launch_mid_atoms(hipStream_t st, int N, const PoseSlot* slots, const 
     return hipErrorInvalidValue;
   const dim3 grid(xcd_plane_grid((N / 2 + 1) / 8, (N / 2 + 1) % 8, (int)ceil_div(nslots, group)));
   CDK_DISPATCH_N(N, {
-    if constexpr (PL::N == 64)
-      hipLaunchKernelGGL((products == kAtomF16x3 ? k_mid_atoms<PL, kAtomF16x3>
-                          : products == kAtomF16 ? k_mid_atoms<PL, kAtomF16>
-                                                 : k_mid_atoms<PL, kAtomF32>),
-                         grid, dim3(kBlock), 0, st, slots, ligs, pad_atoms, wv, wq, ag, astride, meta, nslots, group,
-                         P3, T2, invG, tw);
+    if constexpr (PL::N == 64) {
+      // astride: the largest atom count of the search
+      if (products == kAtomF16x3 && astride <= AtomTab::ROWS) {
+        constexpr int ITEMS = (PL::ZH + AtomTab::NP - 1) / AtomTab::NP;
+        const dim3 g(xcd_plane_grid(ITEMS / 8, ITEMS % 8, (int)ceil_div(nslots, group)));
+        hipLaunchKernelGGL(k_mid_atoms_x3<PL>, g, dim3(128 * AtomTab::NP), 0, st, slots, ligs, pad_atoms, wv, wq, ag,
+                           astride, meta, nslots, group, P3, T2, invG, tw);
+      } else {
+        hipLaunchKernelGGL((products == kAtomF16x3 ? k_mid_atoms<PL, kAtomF16x3>
+                            : products == kAtomF16 ? k_mid_atoms<PL, kAtomF16>
+                                                   : k_mid_atoms<PL, kAtomF32>),
+                           grid, dim3(kBlock), 0, st, slots, ligs, pad_atoms, wv, wq, ag, astride, meta, nslots, group, P3,
+                           T2, invG, tw);
+      }
+    }
     if constexpr (PL::N == 96 || PL::N == 128) {
       constexpr int NB = PL::N / 32;
       const dim3 gf(xcd_plane_grid(PL::ZH / 8, PL::ZH % 8, NB * (int)ceil_div(nslots, group)));

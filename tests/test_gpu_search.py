@@ -521,3 +521,33 @@ def test_large_grids_vs_oracle(ctx, name):
         assert stats.get("exact", 0) >= 3
     lig.close()
     prot.close()
+
+
+@pytest.mark.parametrize("natom", [1, 8, 9, 83, 84, 85])
+def test_atom_form_64_table_edges(ctx, p64, natom):
+    """64^3 atom form around the atom count its operand table holds (84) and
+    one 8-entry step (8, 9): against the FP64 oracle, and bit-identical to the
+    same poses in a batch with an 85-atom ligand, which the table does not
+    hold."""
+    say("atom form table edge natom=%d" % natom)
+    g, prot = p64
+    x, q, e, r = cdk.synth_ligand(700 + natom, natom)
+    lig = cdk.Ligand(prot, q, e, r)
+    quats = cdk.QuaternionUniformSampling(cdk.Rng(17), 6)
+    ctx.set_option("pipeline", 2)
+    try:
+        E, idx, mc = cdk.search(ctx, prot, lig, x[None], quats)
+        xb, qb, eb, rb = cdk.synth_ligand(799, 85)
+        big = cdk.Ligand(prot, qb, eb, rb)
+        b = cdk.Batch(ctx, prot)
+        b.add(big, xb[None], quats)
+        b.add(lig, x[None], quats)
+        b.run()
+        Eb, ib, mb = b.results(1)
+        b.close()
+    finally:
+        ctx.set_option("pipeline", -1)
+    assert np.array_equal(E.view(np.uint32), Eb.view(np.uint32)) and np.array_equal(idx, ib)
+    assert np.array_equal(mc.view(np.uint32), mb.view(np.uint32))
+    prob = orc.PoseProblem(g["values"], g["radii"], g["spacing"], q, e, r)
+    check_search(prob, x[None], quats[:2], E[:, :2], idx[:, :2], mc[:, :2])
