@@ -239,3 +239,24 @@ def test_callers_at_bench_sizes(ctx):
     finally:
         lig.close()
         prot.close()
+
+
+@pytest.mark.parametrize("natom,nprobe,lj_cut,el_cut", [(0, 1, 8.0, 12.0), (1, 4, 8.0, 12.0), (64, 5, 3.0, 5.0),
+                                                       (257, 8, 6.0, 4.0), (300, 13, 2.0, 9.0)])
+def test_grid_builder_edges(ctx, natom, nprobe, lj_cut, el_cut):
+    """The builder's cube-by-cube atom selection at the edges of its 64-atom
+    batches, 256-atom tiles and probe groups, cutoffs in either order, atoms
+    outside the box and one on a grid point: bit for bit the oracle's."""
+    n, h, box = 48, 0.375, 18.0
+    rs = np.random.default_rng(natom + nprobe)
+    x = rs.uniform(-4.0, box + 4.0, (natom, 3))
+    q, e, r = rs.normal(0, 0.3, natom), rs.uniform(0.05, 0.25, natom), rs.uniform(1.2, 2.2, natom)
+    radii = np.linspace(1.0, 2.5, nprobe).astype(np.float32)
+    mid, ln = np.full(3, box / 2, np.float32), np.full(3, (n - 1) * h, np.float32)
+    gm = (np.float32(mid[0]) - np.float32(ln[0]) / np.float32(2)).astype(np.float64)
+    if natom:
+        x[0] = gm + np.array([5, 11, 30]) * h
+    built = cdk.Protein.build(ctx, x, q, e, r, radii, n, h, mid, ln, lj_cut, el_cut)
+    ref = orc.build_grids(x, q, e, r, radii, n, np.full(3, gm), h, lj_cut, el_cut)
+    assert np.array_equal(built.grids(), ref)
+    built.close()
