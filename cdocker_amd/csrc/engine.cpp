@@ -1350,34 +1350,60 @@ int generate_conformers(Context& ctx, int natom, const double* coords, int nroto
   for (int r = 0; r < nrotor; ++r)
     for (int k = 0; k < 4; ++k)
       if (rotors[r * 4 + k] < 0 || rotors[r * 4 + k] >= natom) throw Error(kErrInvalid, "rotor atom out of range");
-  std::vector<double> x(coords, coords + (size_t)natom * 3);
+  const size_t per = (size_t)natom * 3;
+  std::vector<double> x(coords, coords + per);
   std::vector<int> rot(rotors, rotors + (size_t)nrotor * 4);
-  std::vector<unsigned char> mv(moving, moving + (size_t)nrotor * natom);
-  std::vector<unsigned char> ex(exclude, exclude + (size_t)natom * natom);
-  DevBuf d_x, d_rot, d_mv, d_ex, d_out, d_ok;
+  const int rw = (nrotor + 63) / 64, ew = (natom + 63) / 64;
+  std::vector<unsigned long long> mv((size_t)rw * natom, 0ull), ex((size_t)natom * ew, 0ull);
+  for (int r = 0; r < nrotor; ++r)
+    for (int a = 0; a < natom; ++a)
+      if (moving[(size_t)r * natom + a]) mv[(size_t)(r / 64) * natom + a] |= 1ull << (r % 64);
+  for (int a = 0; a < natom; ++a)
+    for (int b = 0; b < natom; ++b)
+      if (exclude[(size_t)a * natom + b]) ex[(size_t)a * ew + b / 64] |= 1ull << (b % 64);
+  DevBuf d_x, d_rot, d_mv, d_ex, d_out, d_ok, d_list, d_kept, d_trial;
   upload(ctx, d_x, x);
   upload(ctx, d_rot, rot);
   upload(ctx, d_mv, mv);
   upload(ctx, d_ex, ex);
-  const size_t per = (size_t)natom * 3;
-  d_out.ensure((size_t)ntrial * per * sizeof(double));
-  d_ok.ensure((size_t)ntrial * sizeof(int));
-  hip_check(launch_conformers(ctx.stream, natom, d_x.as<double>(), nrotor, d_rot.as<int>(),
-                              d_mv.as<unsigned char>(), d_ex.as<unsigned char>(), ntrial, seed, clash_dist,
-                              d_out.as<double>(), d_ok.as<int>()),
-            "conformers");
-  std::vector<int> ok(ntrial);
-  std::vector<double> all((size_t)ntrial * per);
-  hip_check(hipMemcpyAsync(ok.data(), d_ok.p, ok.size() * sizeof(int), hipMemcpyDeviceToHost, ctx.stream), "ok D2H");
-  hip_check(hipMemcpyAsync(all.data(), d_out.p, all.size() * sizeof(double), hipMemcpyDeviceToHost, ctx.stream),
-            "conformers D2H");
-  hip_check(hipStreamSynchronize(ctx.stream), "conformers sync");
-  int kept = 0;
-  for (int t = 0; t < ntrial && kept < max_keep; ++t) {
-    if (!ok[t]) continue;
-    std::memcpy(out + (size_t)kept * per, all.data() + (size_t)t * per, per * sizeof(double));
-    if (trial_index) trial_index[kept] = t;
-    ++kept;
+  // Trials run a set at a time and stop once enough have passed: the kept
+  // ones are the first max_keep in trial order, so later trials cannot
+  // matter.  A first set of 4 096 (four wavefronts per SIMD) takes hardly
+  // longer than one of a few; the next sets follow the share that passed.
+  int kept = 0, done = 0;
+  int set = std::min(ntrial, std::max(4096, max_keep));
+  while (done < ntrial && kept < max_keep) {
+    const int need = std::min(max_keep - kept, set);
+    d_out.ensure((size_t)set * per * sizeof(double));
+    d_ok.ensure((size_t)set * sizeof(int));
+    d_list.ensure((size_t)(need + 1) * sizeof(int));
+    d_kept.ensure((size_t)need * per * sizeof(double));
+    d_trial.ensure((size_t)need * sizeof(int));
+    int* d_count = d_list.as<int>() + need;
+    hip_check(launch_conformers(ctx.stream, natom, d_x.as<double>(), nrotor, d_rot.as<int>(),
+                                d_mv.as<unsigned long long>(), d_ex.as<unsigned long long>(), done, set, seed,
+                                clash_dist, d_out.as<double>(), d_ok.as<int>()),
+              "conformers");
+    hip_check(launch_keep_conformers(ctx.stream, natom, done, set, d_ok.as<int>(), d_out.as<double>(), need,
+                                     d_list.as<int>(), d_count, d_kept.as<double>(), d_trial.as<int>()),
+              "conformers kept");
+    int n = 0;
+    hip_check(hipMemcpyAsync(&n, d_count, sizeof(int), hipMemcpyDeviceToHost, ctx.stream), "count D2H");
+    hip_check(hipStreamSynchronize(ctx.stream), "conformers sync");
+    if (n > 0) {
+      hip_check(hipMemcpyAsync(out + (size_t)kept * per, d_kept.p, (size_t)n * per * sizeof(double),
+                               hipMemcpyDeviceToHost, ctx.stream),
+                "conformers D2H");
+      if (trial_index)
+        hip_check(hipMemcpyAsync(trial_index + kept, d_trial.p, (size_t)n * sizeof(int), hipMemcpyDeviceToHost,
+                                 ctx.stream),
+                  "trials D2H");
+      hip_check(hipStreamSynchronize(ctx.stream), "conformers sync");
+    }
+    kept += n;
+    done += set;
+    const double pass = (double)std::max(kept, 1) / done;
+    set = (int)std::min<double>(ntrial - done, std::max(4096.0, 1.25 * (max_keep - kept) / pass));
   }
   return kept;
 }

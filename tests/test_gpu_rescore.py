@@ -260,3 +260,23 @@ def test_grid_builder_edges(ctx, natom, nprobe, lj_cut, el_cut):
     ref = orc.build_grids(x, q, e, r, radii, n, np.full(3, gm), h, lj_cut, el_cut)
     assert np.array_equal(built.grids(), ref)
     built.close()
+
+
+@pytest.mark.parametrize("natom,ntrial,keep,clash", [(3, 5, 5, 1.2), (40, 5000, 700, 1.2), (70, 300, 300, 0.6),
+                                                    (64, 70, 10, 0.9)])
+def test_conformer_sets_and_words(ctx, natom, ntrial, keep, clash):
+    """Conformer trials at the edges of the 64-bit rotor and atom words (70
+    atoms and 67 rotors, 64 atoms), no rotor, and over more than one set of
+    trials (5 000 with 700 wanted): trials and coordinates as the oracle's."""
+    x, q, e, r = cdk.synth_ligand(300 + natom, natom)
+    rot, mv, ex = workloads.chain_topology(natom) if natom > 3 else (
+        np.zeros((0, 4), np.int32), np.zeros((0, natom), np.uint8), np.ones((natom, natom), np.uint8))
+    conf, trial = cdk.generate_conformers(ctx, x, rot, mv, ex, ntrial, 9, clash, max_keep=keep)
+    if natom > 3:
+        ref, ok = orc.conformers(x.astype(np.float64), rot, mv, ex, ntrial, 9, clash)
+    else:
+        ref, ok = np.repeat(x[None].astype(np.float64), ntrial, 0), np.ones(ntrial, bool)
+    want = np.flatnonzero(ok)[:keep]
+    say("conformers natom=%d: %d of %d pass" % (natom, int(np.sum(ok)), ntrial))
+    assert len(want) > 0 and np.array_equal(trial, want)
+    assert np.abs(conf - ref[want]).max() < 1e-9
