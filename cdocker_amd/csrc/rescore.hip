@@ -49,14 +49,23 @@ __device__ __forceinline__ AtomTerm atom_term(const float* __restrict__ grid, in
   const float* pv = pch >= 0 ? grid + (size_t)pch * G + base : nullptr;
   const float* pe = grid + (size_t)ech * G + base;
   double e = 0.0, d0 = 0.0, d1 = 0.0, d2 = 0.0;
+  // The corners' grid values, the two of a z edge in one load (4-byte aligned):
+  // each lane's cell lies in lines of its own, so a load instruction costs its
+  // lanes one by one and half the instructions take half the time.
+  float fe[8], fv[8];
+#pragma unroll
+  for (int c = 0; c < 8; c += 2) {
+    const size_t off = ((size_t)(c >> 2) * N + ((c >> 1) & 1)) * N;
+    __builtin_memcpy(fe + c, pe + off, 8);
+    if (pv) __builtin_memcpy(fv + c, pv + off, 8);
+  }
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
     const int dx = c >> 2, dy = (c >> 1) & 1, dz = c & 1;
-    const size_t off = ((size_t)dx * N + dy) * N + dz;
     const double X = dx ? f[0] : 1.0 - f[0], Y = dy ? f[1] : 1.0 - f[1], Z = dz ? f[2] : 1.0 - f[2];
     const double sx = dx ? 1.0 : -1.0, sy = dy ? 1.0 : -1.0, sz = dz ? 1.0 : -1.0;
-    double v = wq * (double)pe[off];
-    if (pv) v += wv * (double)pv[off];
+    double v = wq * (double)fe[c];
+    if (pv) v += wv * (double)fv[c];
     e += X * Y * Z * v;
     d0 += sx * Y * Z * v;
     d1 += X * sy * Z * v;
@@ -122,104 +131,196 @@ __global__ __launch_bounds__(256) void k_rescore(int npose, int natom, const dou
 // rotates by sr about tau (Rodrigues).  A trial that lowers E + penalty is
 // kept and both steps grow by 1.2 (capped), otherwise they halve.  Atoms off
 // the grid add `penalty` each, so a pose cannot lower its score by leaving.
-__device__ double pose_score(const double* __restrict__ r, int natom, const int* __restrict__ pch,
-                             const float* __restrict__ wv, const float* __restrict__ wq,
-                             const float* __restrict__ grid, int N, int ech, double g0, double g1, double g2,
-                             double inv_h, double penalty, double* F, double* tau, const double* c) {
-  const int lane = threadIdx.x & 63;
-  double e = 0.0, f[3] = {0, 0, 0}, t[3] = {0, 0, 0};
-  for (int a = lane; a < natom; a += 64) {
-    const double x = r[a * 3 + 0], y = r[a * 3 + 1], z = r[a * 3 + 2];
-    const AtomTerm at = atom_term(grid, N, pch[a], ech, (double)wv[a], (double)wq[a], x, y, z, g0, g1, g2, inv_h);
-    e += at.inside ? at.e : penalty;
-    const double fx = -at.g[0], fy = -at.g[1], fz = -at.g[2];
-    f[0] += fx;
-    f[1] += fy;
-    f[2] += fz;
-    const double dx = x - c[0], dy = y - c[1], dz = z - c[2];
-    t[0] += dy * fz - dz * fy;
-    t[1] += dz * fx - dx * fz;
-    t[2] += dx * fy - dy * fx;
+// ---- sums over the wavefront, several at a time -----------------------------
+// Eight lane values v[0..7] -> their eight wavefront sums, sum k on the lanes
+// whose bits 5, 4, 3 spell k: at each of the first three halvings a lane keeps
+// half of the values and takes its partner's, so the eight sums cost 10 adds
+// and exchanges instead of 48.  Every sum adds the same pairs as wave_sum's
+// butterfly (lanes 32 apart, then 16, 8, 4, 2, 1): the same bits.
+struct F64Pair {
+  double a, b;
+};
+__device__ __forceinline__ F64Pair swap32(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return {__longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])),
+          __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]))};
+}
+__device__ __forceinline__ F64Pair swap16(double a, double b) {
+  const unsigned long long x = (unsigned long long)__double_as_longlong(a), y = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+  return {__longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])),
+          __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]))};
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// v of the lane 4 away (lane ^ 4): half-row mirror (^ 7), then quad reversal (^ 3).
+__device__ __forceinline__ double xor4(double v) { return dpp64<0x1B>(dpp64<0x141>(v)); }
+
+__device__ __forceinline__ double wave_sum8(const double (&v)[8]) {
+  double h[4], q[2];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const F64Pair p = swap32(v[k], v[k + 4]);
+    h[k] = p.a + p.b;
   }
-  for (int k = 0; k < 3; ++k) {
-    F[k] = wave_sum(f[k]);
-    tau[k] = wave_sum(t[k]);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const F64Pair p = swap16(h[k], h[k + 2]);
+    q[k] = p.a + p.b;
   }
-  return wave_sum(e);
+  const bool up = (threadIdx.x & 8) != 0;
+  const double keep = up ? q[1] : q[0], give = up ? q[0] : q[1];
+  double s = keep + dpp64<0x128>(give);  // row rotation by 8: lane ^ 8
+  s += xor4(s);
+  s += dpp64<0x4E>(s);  // quad permutation 2 3 0 1: lane ^ 2
+  s += dpp64<0xB1>(s);  // quad permutation 1 0 3 2: lane ^ 1
+  return s;
 }
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// One 64-thread workgroup per pose; the pose and the trial pose live in LDS
-// (2 * natom * 3 doubles), so every lane sees the others' writes in order.
+// Lane sums of the force, the torque and the score of one pose: v[0..2] F,
+// v[3..5] tau, v[6] E (penalty for an atom off the grid), v[7] = 0.
+struct PoseTerm {
+  double x, y, z;  // position
+  double wv, wq;
+  int pch;
+};
+__device__ __forceinline__ void add_terms(const PoseTerm& p, const float* __restrict__ grid, int N, int ech, double g0,
+                                          double g1, double g2, double inv_h, double penalty, const double (&c)[3],
+                                          double (&v)[8]) {
+  const AtomTerm at = atom_term(grid, N, p.pch, ech, p.wv, p.wq, p.x, p.y, p.z, g0, g1, g2, inv_h);
+  v[6] += at.inside ? at.e : penalty;
+  const double fx = -at.g[0], fy = -at.g[1], fz = -at.g[2];
+  v[0] += fx;
+  v[1] += fy;
+  v[2] += fz;
+  const double dx = p.x - c[0], dy = p.y - c[1], dz = p.z - c[2];
+  v[3] += dy * fz - dz * fy;
+  v[4] += dz * fx - dx * fz;
+  v[5] += dx * fy - dy * fx;
+}
+
+// One 64-thread workgroup per pose, atoms strided over the lanes (AL per lane,
+// in registers).
+//
+// What bounds it: one wavefront per pose and a serial chain of `steps` score
+// evaluations, so time is the chain's latency.  Keeping each lane's atoms,
+// channels and weights in registers takes the LDS round trips and their
+// global reloads out of it; the seven sums of an evaluation cost ten adds
+// (wave_sum8) instead of 42 rounds through the LDS crossbar; the two norms and
+// the six quotients that follow are each one square root and one division,
+// on the lanes that hold the sums.  What is left per step is the latency of
+// the grid gather and of the FP64 terms.  Measured, 1 000 poses of 40 atoms,
+// 50 steps: 251 -> 194 us, and 117 us with the corner pairs of atom_term.
+template <int AL>
 __global__ __launch_bounds__(64) void k_refine(int npose, int natom, double* __restrict__ coords,
                                                const int* __restrict__ pch, const float* __restrict__ wv,
                                                const float* __restrict__ wq, const float* __restrict__ grid, int N,
                                                int ech, double g0, double g1, double g2, double inv_h, int steps,
                                                double penalty, double* __restrict__ energy) {
-  extern __shared__ double sm[];
   const int pose = blockIdx.x;
   const int lane = threadIdx.x;
   if (pose >= npose) return;
   double* gr = coords + (size_t)pose * natom * 3;
-  double* r = sm;
-  double* q = sm + natom * 3;
-  for (int i = lane; i < natom * 3; i += 64) r[i] = gr[i];
-  wave_sync();
-  double c[3];
-  for (int k = 0; k < 3; ++k) {
-    double s = 0.0;
-    for (int a = lane; a < natom; a += 64) s += r[a * 3 + k];
-    c[k] = wave_sum(s) / (double)natom;
+  PoseTerm r[AL], q[AL];
+#pragma unroll
+  for (int u = 0; u < AL; ++u) {
+    const int a = lane + 64 * u;
+    r[u] = PoseTerm{0.0, 0.0, 0.0, 0.0, 0.0, -1};
+    if (a < natom) r[u] = PoseTerm{gr[a * 3 + 0], gr[a * 3 + 1], gr[a * 3 + 2], (double)wv[a], (double)wq[a], pch[a]};
+    q[u] = r[u];
   }
-  double F[3], tau[3];
-  double e = pose_score(r, natom, pch, wv, wq, grid, N, ech, g0, g1, g2, inv_h, penalty, F, tau, c);
+  double c[3];
+  {
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < AL; ++u)
+      if (lane + 64 * u < natom) {
+        v[0] += r[u].x;
+        v[1] += r[u].y;
+        v[2] += r[u].z;
+      }
+    const double s = wave_sum8(v);
+    for (int k = 0; k < 3; ++k) c[k] = lane_value(s, 8 * k) / (double)natom;
+  }
+  // this lane's sum among F (0..2), tau (3..5) and E (6), and all of them
+  auto score = [&](const PoseTerm (&p)[AL], const double (&cc)[3]) {
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < AL; ++u)
+      if (lane + 64 * u < natom) add_terms(p[u], grid, N, ech, g0, g1, g2, inv_h, penalty, cc, v);
+    return wave_sum8(v);
+  };
+  const int mine = lane >> 3;  // which sum this lane holds
+  double s = score(r, c);
+  double e = lane_value(s, 48);
   double st = 0.1, sr = 0.02;
   const double st_max = 0.5, sr_max = 0.1;
   for (int it = 0; it < steps; ++it) {
-    const double fn = sqrt(F[0] * F[0] + F[1] * F[1] + F[2] * F[2]);
-    const double tn = sqrt(tau[0] * tau[0] + tau[1] * tau[1] + tau[2] * tau[2]);
+    // |F| on the lanes of F, |tau| on the others
+    const bool rot = mine >= 3;
+    const double n0 = lane_value(s, 0), n1 = lane_value(s, 8), n2 = lane_value(s, 16);
+    const double m0 = lane_value(s, 24), m1 = lane_value(s, 32), m2 = lane_value(s, 40);
+    const double v0 = rot ? m0 : n0, v1 = rot ? m1 : n1, v2 = rot ? m2 : n2;
+    const double norm = sqrt(v0 * v0 + v1 * v1 + v2 * v2);
+    const double fn = lane_value(norm, 0), tn = lane_value(norm, 24);
     if (fn == 0.0 && tn == 0.0) break;
-    double d[3], ax[3];
-    for (int k = 0; k < 3; ++k) {
-      d[k] = fn > 0.0 ? st * F[k] / fn : 0.0;
-      ax[k] = tn > 0.0 ? tau[k] / tn : 0.0;
-    }
+    // d = st F / |F|, axis = tau / |tau|
+    const double num = rot ? s : st * s;
+    const double quo = norm > 0.0 ? num / norm : 0.0;
+    const double d[3] = {lane_value(quo, 0), lane_value(quo, 8), lane_value(quo, 16)};
+    const double ax[3] = {lane_value(quo, 24), lane_value(quo, 32), lane_value(quo, 40)};
     const double th = tn > 0.0 ? sr : 0.0;
-    const double ct = cos(th), sn = sin(th);
-    for (int a = lane; a < natom; a += 64) {
-      const double v0 = r[a * 3 + 0] - c[0], v1 = r[a * 3 + 1] - c[1], v2 = r[a * 3 + 2] - c[2];
+    double ct, sn;
+    sincos(th, &sn, &ct);
+#pragma unroll
+    for (int u = 0; u < AL; ++u) {
+      const double v0 = r[u].x - c[0], v1 = r[u].y - c[1], v2 = r[u].z - c[2];
       const double kd = ax[0] * v0 + ax[1] * v1 + ax[2] * v2;
       const double cx = ax[1] * v2 - ax[2] * v1, cy = ax[2] * v0 - ax[0] * v2, cz = ax[0] * v1 - ax[1] * v0;
-      q[a * 3 + 0] = c[0] + d[0] + v0 * ct + cx * sn + ax[0] * kd * (1.0 - ct);
-      q[a * 3 + 1] = c[1] + d[1] + v1 * ct + cy * sn + ax[1] * kd * (1.0 - ct);
-      q[a * 3 + 2] = c[2] + d[2] + v2 * ct + cz * sn + ax[2] * kd * (1.0 - ct);
+      q[u].x = c[0] + d[0] + v0 * ct + cx * sn + ax[0] * kd * (1.0 - ct);
+      q[u].y = c[1] + d[1] + v1 * ct + cy * sn + ax[1] * kd * (1.0 - ct);
+      q[u].z = c[2] + d[2] + v2 * ct + cz * sn + ax[2] * kd * (1.0 - ct);
     }
-    wave_sync();
     const double cn[3] = {c[0] + d[0], c[1] + d[1], c[2] + d[2]};
-    double F2[3], tau2[3];
-    const double e2 = pose_score(q, natom, pch, wv, wq, grid, N, ech, g0, g1, g2, inv_h, penalty, F2, tau2, cn);
-    if (e2 < e) {  // wave-uniform: every lane holds the reduced sums
-      for (int i = lane; i < natom * 3; i += 64) r[i] = q[i];
+    const double s2 = score(q, cn);
+    const double e2 = lane_value(s2, 48);
+    if (e2 < e) {  // wave-uniform
+#pragma unroll
+      for (int u = 0; u < AL; ++u) r[u] = q[u];
       e = e2;
-      for (int k = 0; k < 3; ++k) {
-        c[k] = cn[k];
-        F[k] = F2[k];
-        tau[k] = tau2[k];
-      }
+      s = s2;
+      for (int k = 0; k < 3; ++k) c[k] = cn[k];
       st = fmin(st * 1.2, st_max);
       sr = fmin(sr * 1.2, sr_max);
     } else {
       st *= 0.5;
       sr *= 0.5;
     }
-    wave_sync();
   }
-  for (int i = lane; i < natom * 3; i += 64) gr[i] = r[i];
+#pragma unroll
+  for (int u = 0; u < AL; ++u) {
+    const int a = lane + 64 * u;
+    if (a < natom) {
+      gr[a * 3 + 0] = r[u].x;
+      gr[a * 3 + 1] = r[u].y;
+      gr[a * 3 + 2] = r[u].z;
+    }
+  }
   if (lane == 0) energy[pose] = e;
 }
 
@@ -259,9 +360,10 @@ hipError_t launch_refine(hipStream_t st, int npose, int natom, double* coords, c
                          const float* wq, const float* grid, int N, int ech, const double* gmin, double h, int steps,
                          double penalty, double* energy) {
   if (npose <= 0) return hipSuccess;
-  const size_t lds = (size_t)natom * 6 * sizeof(double);
-  hipLaunchKernelGGL(k_refine, dim3((unsigned)npose), dim3(64), lds, st, npose, natom, coords, pch, wv, wq, grid, N,
-                     ech, gmin[0], gmin[1], gmin[2], 1.0 / h, steps, penalty, energy);
+  if (natom <= 0 || natom > 64 * 8) return hipErrorInvalidValue;
+  auto* k = natom <= 64 ? k_refine<1> : natom <= 128 ? k_refine<2> : natom <= 256 ? k_refine<4> : k_refine<8>;
+  hipLaunchKernelGGL(k, dim3((unsigned)npose), dim3(64), 0, st, npose, natom, coords, pch, wv, wq, grid, N, ech,
+                     gmin[0], gmin[1], gmin[2], 1.0 / h, steps, penalty, energy);
   return hipGetLastError();
 }
 

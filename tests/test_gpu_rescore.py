@@ -280,3 +280,28 @@ def test_conformer_sets_and_words(ctx, natom, ntrial, keep, clash):
     say("conformers natom=%d: %d of %d pass" % (natom, int(np.sum(ok)), ntrial))
     assert len(want) > 0 and np.array_equal(trial, want)
     assert np.abs(conf - ref[want]).max() < 1e-9
+
+
+@pytest.mark.parametrize("natom", [1, 63, 64, 65, 128, 129, 257, 512])
+def test_refine_atom_counts(ctx, p48, natom):
+    """The descent's register forms at their atom-count edges: every pose ends
+    rigid (pair distances kept to 1e-9 A) and at the energy the FP64 rescoring
+    gives it, no higher than it started (off-grid atoms counted as the
+    penalty)."""
+    g, prot = p48
+    rs = np.random.default_rng(natom)
+    d = rs.normal(size=(natom, 3))
+    x = 4.0 * d / np.linalg.norm(d, axis=1, keepdims=True) * rs.uniform(0, 1, (natom, 1)) ** (1 / 3)
+    _, q, e, r = cdk.synth_ligand(natom, natom)
+    lig = cdk.Ligand(prot, q, e, r)
+    poses = x[None] + rs.uniform(-6.0, 6.0, (5, 1, 3)) + np.asarray(g["mid"], np.float64)
+    out, en = cdk.refine_poses(prot, lig, poses, steps=15, off_grid_penalty=10.0)
+    e0, _, in0 = cdk.rescore_poses(prot, lig, poses)
+    e1, _, in1 = cdk.rescore_poses(prot, lig, out)
+    scale = np.abs(q).sum() * 20.0 + 1.0
+    assert np.abs(en - (e1 + 10.0 * (natom - in1))).max() <= 1e-12 * scale
+    assert (en <= e0 + 10.0 * (natom - in0) + 1e-12 * scale).all()
+    i, j = rs.integers(0, natom, 50), rs.integers(0, natom, 50)
+    dist = lambda p: np.linalg.norm(p[:, i] - p[:, j], axis=-1)  # noqa: E731
+    assert np.abs(dist(out) - dist(poses)).max() < 1e-9
+    lig.close()
