@@ -283,8 +283,7 @@ int cdk_protein_grids(cdk_protein* p, float* values) {
     cdk::Context& ctx = *p->p.ctx;
     std::lock_guard<std::mutex> lk(ctx.mu);
     cdk::hip_check(hipSetDevice(ctx.device), "hipSetDevice");
-    cdk::hip_check(hipMemcpy(values, p->p.grid.p, (size_t)p->p.nch * p->p.G() * sizeof(float), hipMemcpyDeviceToHost),
-                   "grids D2H");
+    cdk::CallScratch(ctx).out(values, p->p.grid.p, (size_t)p->p.nch * p->p.G() * sizeof(float));
   });
 }
 
@@ -299,15 +298,15 @@ int cdk_protein_spectrum(cdk_protein* p, int channel, float* out) {
     cdk::Context& c = *p->p.ctx;
     std::lock_guard<std::mutex> lk(c.mu);
     const size_t H = p->p.H();
-    d2h(c, out, p->p.spec.as<float2>() + (size_t)channel * H, H * sizeof(float2));
-    sync(c);
+    cdk::hip_check(hipSetDevice(c.device), "hipSetDevice");
+    cdk::CallScratch(c).out(out, p->p.spec.as<float2>() + (size_t)channel * H, H * sizeof(float2));
   });
 }
 
 int cdk_protein_bytes(cdk_protein* p, int64_t* bytes) {
   return guard([&] {
     require(p && bytes, "NULL argument");
-    *bytes = (int64_t)(p->p.grid.cap + p->p.spec.cap + p->p.spec_lb.cap + p->p.spec_kz.cap + p->p.spec_mf.cap);
+    *bytes = (int64_t)p->p.all.cap;
   });
 }
 
@@ -361,12 +360,7 @@ int cdk_search(cdk_context* ctx, cdk_protein* p, const cdk_ligand* l, int nconf,
     j.nquat = nquat;
     j.quats = quats;
     j.shared_quats = shared_quats != 0;
-    std::vector<cdk::PoseResults> out;
-    cdk::run_search(*ctx->c, p->p, {j}, (cdk::Engine)engine, out);
-    const size_t n = (size_t)nconf * nquat;
-    std::memcpy(energy, out[0].energy.data(), n * sizeof(float));
-    if (index) std::memcpy(index, out[0].index.data(), n * 3 * sizeof(int));
-    if (mincoor) std::memcpy(mincoor, out[0].mincoor.data(), n * 3 * sizeof(float));
+    cdk::run_search(*ctx->c, p->p, j, (cdk::Engine)engine, energy, index, mincoor);
   });
 }
 

@@ -58,8 +58,9 @@ Context::~Context() {
   if (stream) (void)hipStreamSynchronize(stream);
   if (stream_z) (void)hipStreamSynchronize(stream_z);
   for (auto& kv : twiddles) delete kv.second;
-  if (h_keys) (void)hipHostFree(h_keys);
-  if (h_meta) (void)hipHostFree(h_meta);
+  idle.clear();
+  if (call_host) (void)hipHostFree(call_host);
+  for (hipEvent_t e : call_events) (void)hipEventDestroy(e);
   for (hipEvent_t e : set_events) (void)hipEventDestroy(e);
   if (stream_z) (void)hipStreamDestroy(stream_z);
   if (stream) (void)hipStreamDestroy(stream);
@@ -81,24 +82,102 @@ const float2* Context::twiddle(int N) {
   return b->as<float2>();
 }
 
-void Context::ensure_host(size_t nslots) {
-  if (nslots <= h_cap) return;
-  if (h_keys) (void)hipHostFree(h_keys);
-  if (h_meta) (void)hipHostFree(h_meta);
-  h_keys = h_meta = nullptr;
-  hip_check(hipHostMalloc(&h_keys, nslots * sizeof(unsigned long long)), "hipHostMalloc");
-  hip_check(hipHostMalloc(&h_meta, nslots * sizeof(RotMeta)), "hipHostMalloc");
-  h_cap = nslots;
+CallScratch::CallScratch(Context& c) : ctx_(c), exceptions_(std::uncaught_exceptions()) {}
+
+CallScratch::~CallScratch() {
+  if (std::uncaught_exceptions() > exceptions_) (void)hipStreamSynchronize(ctx_.stream);
+  if (ctx_.call_dev.cap > kKeepDev) {
+    (void)hipStreamSynchronize(ctx_.stream);
+    ctx_.call_dev.release();
+  }
+  if (ctx_.call_host_cap > kKeepHost) {
+    (void)hipStreamSynchronize(ctx_.stream);
+    (void)hipHostFree(ctx_.call_host);
+    ctx_.call_host = nullptr;
+    ctx_.call_host_cap = 0;
+  }
+}
+
+char* CallScratch::dev(size_t bytes) {
+  if (bytes > ctx_.call_dev.cap) {
+    hip_check(hipStreamSynchronize(ctx_.stream), "hipStreamSynchronize");
+    ctx_.call_dev.ensure((bytes + 0xffff) & ~(size_t)0xffff);
+  }
+  return ctx_.call_dev.as<char>();
+}
+
+char* CallScratch::host(size_t bytes) {
+  if (bytes > ctx_.call_host_cap) {
+    hip_check(hipStreamSynchronize(ctx_.stream), "hipStreamSynchronize");  // its last transfers
+    if (ctx_.call_host) (void)hipHostFree(ctx_.call_host);
+    ctx_.call_host = nullptr;
+    ctx_.call_host_cap = 0;
+    bytes = (bytes + 0xffff) & ~(size_t)0xffff;
+    // coherent: kernels read and write it in place
+    hip_check(hipHostMalloc(&ctx_.call_host, bytes, hipHostMallocCoherent), "hipHostMalloc");
+    ctx_.call_host_cap = bytes;
+  }
+  return static_cast<char*>(ctx_.call_host);
 }
 
 namespace {
 
-template <class T>
-void upload(Context& ctx, DevBuf& b, const std::vector<T>& v) {
-  b.ensure(std::max<size_t>(v.size(), 1) * sizeof(T));
-  if (!v.empty())
-    hip_check(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, ctx.stream), "upload");
+// Pieces of the copies.  Measured for 9.4 MB: down 336 us in 1 MB pieces (367
+// in 2 MB, 430 in 512 KB, 485 in one, 540 from pageable memory), up 350 us in
+// 2 MB pieces with the spectra after it (387 in 1 MB, 408 in one).
+constexpr size_t kDownPiece = 1ull << 20, kUpPiece = 2ull << 20;
+constexpr size_t kPieceBytes = 16ull << 20;  // of the host arena, all pieces in flight
+constexpr size_t kMaxPieces = kPieceBytes / kDownPiece;
+
+void slot_events(Context& c) {
+  while (c.call_events.size() < kMaxPieces) {
+    hipEvent_t e = nullptr;
+    hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+    c.call_events.push_back(e);
+  }
 }
+
+}  // namespace
+
+void CallScratch::in(void* dev_dst, const void* src, size_t bytes) {
+  if (!bytes) return;
+  slot_events(ctx_);
+  constexpr size_t kSlotBytes = kUpPiece, kSlots = kPieceBytes / kUpPiece;
+  const size_t n = (bytes + kSlotBytes - 1) / kSlotBytes;
+  char* h = host(std::min(n, kSlots) * kSlotBytes);
+  for (size_t i = 0; i < n; ++i) {
+    char* slot = h + (i % kSlots) * kSlotBytes;
+    const size_t o = i * kSlotBytes, len = std::min(kSlotBytes, bytes - o);
+    if (i >= kSlots) hip_check(hipEventSynchronize(ctx_.call_events[i % kSlots]), "upload slot");
+    std::memcpy(slot, static_cast<const char*>(src) + o, len);
+    hip_check(hipMemcpyAsync(static_cast<char*>(dev_dst) + o, slot, len, hipMemcpyHostToDevice, ctx_.stream), "H2D");
+    if (n > kSlots) hip_check(hipEventRecord(ctx_.call_events[i % kSlots], ctx_.stream), "hipEventRecord");
+  }
+}
+
+void CallScratch::out(void* dst, const void* dev_src, size_t bytes) {
+  if (!bytes) return;
+  slot_events(ctx_);
+  constexpr size_t kSlotBytes = kDownPiece, kSlots = kPieceBytes / kDownPiece;
+  const size_t n = (bytes + kSlotBytes - 1) / kSlotBytes;
+  char* h = host(std::min(n, kSlots) * kSlotBytes);
+  auto fetch = [&](size_t i) {
+    const size_t o = i * kSlotBytes, len = std::min(kSlotBytes, bytes - o);
+    hip_check(hipMemcpyAsync(h + (i % kSlots) * kSlotBytes, static_cast<const char*>(dev_src) + o, len,
+                             hipMemcpyDeviceToHost, ctx_.stream),
+              "D2H");
+    hip_check(hipEventRecord(ctx_.call_events[i % kSlots], ctx_.stream), "hipEventRecord");
+  };
+  for (size_t i = 0; i < std::min(n, kSlots); ++i) fetch(i);
+  for (size_t i = 0; i < n; ++i) {
+    const size_t o = i * kSlotBytes, len = std::min(kSlotBytes, bytes - o);
+    hip_check(hipEventSynchronize(ctx_.call_events[i % kSlots]), "download slot");
+    std::memcpy(static_cast<char*>(dst) + o, h + (i % kSlots) * kSlotBytes, len);
+    if (i + kSlots < n) fetch(i + kSlots);
+  }
+}
+
+namespace {
 
 void protein_setup(Protein& p, int nch, int N, float h, const float* mid, const float* len, const float* radii) {
   if (nch < 2 || nch > kMaxCh) throw Error(kErrInvalid, "number of grids must be in [2, 16]");
@@ -112,7 +191,17 @@ void protein_setup(Protein& p, int nch, int N, float h, const float* mid, const 
     p.len[k] = len ? len[k] : (float)(N - 1) * h;
   }
   p.radii.assign(radii, radii + (nch - 1));
-  p.grid.ensure((size_t)nch * p.G() * sizeof(float));
+  const size_t H = (size_t)nch * p.H() * sizeof(float2);
+  Layout l;
+  const size_t grid = l.add((size_t)nch * p.G() * sizeof(float)), spec = l.add(H), lb = l.add(H);
+  const size_t kz = col_supported(N) ? l.add(H) : 0, mf = atoms_supported(N) ? l.add(H) : 0;
+  p.all.ensure(l.end);
+  char* base = p.all.as<char>();
+  p.grid.p = base + grid;
+  p.spec.p = base + spec;
+  p.spec_lb.p = base + lb;
+  if (kz) p.spec_kz.p = base + kz;
+  if (mf) p.spec_mf.p = base + mf;
 }
 
 // Forward R2C of every channel (NoMini:177-199) plus the copies the fused
@@ -120,20 +209,15 @@ void protein_setup(Protein& p, int nch, int N, float h, const float* mid, const 
 // edge 64).
 void protein_spectra(Protein& p) {
   Context& ctx = *p.ctx;
-  const size_t H = p.H();
-  p.spec.ensure((size_t)p.nch * H * sizeof(float2));
   hip_check(launch_r2c_3d(ctx.stream, p.N, p.grid.as<float>(), p.spec.as<float2>(), p.nch, ctx.twiddle(p.N)),
             "protein R2C");
-  p.spec_lb.ensure((size_t)p.nch * H * sizeof(float2));
   hip_check(launch_to_line_blocks(ctx.stream, p.N, p.spec.as<float2>(), p.spec_lb.as<float2>(), p.nch),
             "protein spectra line blocks");
   if (col_supported(p.N)) {
-    p.spec_kz.ensure((size_t)p.nch * H * sizeof(float2));
     hip_check(launch_to_kz_blocks(ctx.stream, p.N, p.spec.as<float2>(), p.spec_kz.as<float2>(), p.nch),
               "protein spectra kz blocks");
   }
   if (atoms_supported(p.N)) {
-    p.spec_mf.ensure((size_t)p.nch * H * sizeof(float2));
     hip_check(launch_to_mfma_blocks(ctx.stream, p.N, p.spec.as<float2>(), p.spec_mf.as<float2>(), p.nch),
               "protein spectra matrix-core blocks");
   }
@@ -146,8 +230,8 @@ void protein_upload(Protein& p, int nch, int N, float h, const float* mid, const
                     const float* values) {
   protein_setup(p, nch, N, h, mid, len, radii);
   Context& ctx = *p.ctx;
-  hip_check(hipMemcpyAsync(p.grid.p, values, (size_t)nch * p.G() * sizeof(float), hipMemcpyHostToDevice, ctx.stream),
-            "protein upload");
+  CallScratch scratch(ctx);
+  scratch.in(p.grid.p, values, (size_t)nch * p.G() * sizeof(float));
   protein_spectra(p);
 }
 
@@ -158,19 +242,24 @@ void protein_build(Protein& p, int natom, const double* xyz, const double* charg
     throw Error(kErrInvalid, "atom count must be >= 0 and probe count in [1, 15]");
   protein_setup(p, nprobe + 1, N, h, mid, len, probe_radii);
   Context& ctx = *p.ctx;
-  std::vector<double> atoms((size_t)std::max(natom, 1) * 6);
+  CallScratch scratch(ctx);
+  Layout l;
+  const size_t o_atoms = l.add((size_t)std::max(natom, 1) * 6 * sizeof(double));
+  const size_t o_probe = l.add((size_t)nprobe * sizeof(double));
+  char* hs = scratch.host(l.end);
+  char* ds = scratch.dev(l.end);
+  double* atoms = reinterpret_cast<double*>(hs + o_atoms);
   for (int i = 0; i < natom; ++i) {
     for (int k = 0; k < 3; ++k) atoms[(size_t)i * 6 + k] = xyz[i * 3 + k];
     atoms[(size_t)i * 6 + 3] = charge[i];
     atoms[(size_t)i * 6 + 4] = radius[i];
     atoms[(size_t)i * 6 + 5] = epsilon[i];
   }
-  std::vector<double> probe(probe_radii, probe_radii + nprobe);
-  DevBuf d_atoms, d_probe;
-  upload(ctx, d_atoms, atoms);
-  upload(ctx, d_probe, probe);
+  std::copy(probe_radii, probe_radii + nprobe, reinterpret_cast<double*>(hs + o_probe));
+  hip_check(hipMemcpyAsync(ds, hs, l.end, hipMemcpyHostToDevice, ctx.stream), "atoms H2D");
   const double gmin[3] = {p.grid_min(0), p.grid_min(1), p.grid_min(2)};
-  hip_check(launch_build_grids(ctx.stream, natom, d_atoms.as<double>(), nprobe, d_probe.as<double>(), N, gmin,
+  hip_check(launch_build_grids(ctx.stream, natom, reinterpret_cast<const double*>(ds + o_atoms), nprobe,
+                               reinterpret_cast<const double*>(ds + o_probe), N, gmin,
                                (double)h, lj_cutoff, elec_cutoff, lj_cap, elec_cap, p.grid.as<float>()),
             "build grids");
   protein_spectra(p);
@@ -972,8 +1061,7 @@ void enqueue_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk,
 Prepared::~Prepared() {
   drop_graph();
   if (h_up) (void)hipHostFree(h_up);
-  if (h_keys) (void)hipHostFree(h_keys);
-  if (h_meta) (void)hipHostFree(h_meta);
+  if (h_res) (void)hipHostFree(h_res);
   if (start) (void)hipEventDestroy(start);
   if (done) (void)hipEventDestroy(done);
 }
@@ -1001,61 +1089,55 @@ void build_search(const Protein& prot, const std::vector<Job>& jobs, Prepared& t
   build_tables(prot, jobs, t);
   for (const Job& j : jobs) t.job_n.push_back(j.npose());
   t.prot = &prot;
+  t.ran = false;
 }
 
 namespace {
 
-// t's tables to the device on the context stream (context lock held).
+// t's tables to the device on the context stream (context lock held): through
+// t's pinned staging in one asynchronous copy (one from pageable memory would
+// hold the host until the stream's earlier work is done).  The staging is
+// rewritten only once that copy is over.
 void upload_tables(Context& ctx, Prepared& t) {
-  if (t.own_staging) {
-    // Pipelined callers: the tables go through this search's own pinned
-    // staging, so the copies are asynchronous (a copy from pageable memory
-    // would hold the host until the stream's earlier work is done).  The
-    // staging is rewritten only after finish_search of this search.
-    struct Part {
-      DevBuf* dst;
-      const void* src;
-      size_t bytes;
-    };
-    const Part parts[7] = {{&t.d_ligs, t.ligs.data(), t.ligs.size() * sizeof(LigandDesc)},
-                           {&t.d_chan, t.chan.data(), t.chan.size() * sizeof(int)},
-                           {&t.d_pad, t.pad.data(), t.pad.size() * sizeof(int)},
-                           {&t.d_wv, t.wv.data(), t.wv.size() * sizeof(float)},
-                           {&t.d_wq, t.wq.data(), t.wq.size() * sizeof(float)},
-                           {&t.d_coords, t.coords.data(), t.coords.size() * sizeof(float)},
-                           {&t.d_slots, t.slots.data(), t.slots.size() * sizeof(PoseSlot)}};
-    size_t off[7], total = 0;
-    for (int i = 0; i < 7; ++i) {
-      off[i] = total;
-      total += (parts[i].bytes + 255) & ~(size_t)255;
-    }
-    if (total > t.h_up_cap) {
-      if (t.h_up) (void)hipHostFree(t.h_up);
-      t.h_up = nullptr;
-      t.h_up_cap = 0;
-      hip_check(hipHostMalloc(&t.h_up, total), "hipHostMalloc");
-      t.h_up_cap = total;
-    }
-    char* h = static_cast<char*>(t.h_up);
-    for (int i = 0; i < 7; ++i) {
-      parts[i].dst->ensure(std::max<size_t>(parts[i].bytes, 4));
-      if (parts[i].bytes == 0) continue;
-      std::memcpy(h + off[i], parts[i].src, parts[i].bytes);
-      hip_check(hipMemcpyAsync(parts[i].dst->p, h + off[i], parts[i].bytes, hipMemcpyHostToDevice, ctx.stream),
-                "upload");
-    }
-  } else {
-    upload(ctx, t.d_ligs, t.ligs);
-    upload(ctx, t.d_chan, t.chan);
-    upload(ctx, t.d_pad, t.pad);
-    upload(ctx, t.d_wv, t.wv);
-    upload(ctx, t.d_wq, t.wq);
-    upload(ctx, t.d_coords, t.coords);
-    upload(ctx, t.d_slots, t.slots);
+  struct Part {
+    DevView* dst;
+    const void* src;
+    size_t bytes, off;
+  };
+  Part parts[7] = {{&t.d_ligs, t.ligs.data(), t.ligs.size() * sizeof(LigandDesc), 0},
+                   {&t.d_chan, t.chan.data(), t.chan.size() * sizeof(int), 0},
+                   {&t.d_pad, t.pad.data(), t.pad.size() * sizeof(int), 0},
+                   {&t.d_wv, t.wv.data(), t.wv.size() * sizeof(float), 0},
+                   {&t.d_wq, t.wq.data(), t.wq.size() * sizeof(float), 0},
+                   {&t.d_coords, t.coords.data(), t.coords.size() * sizeof(float), 0},
+                   {&t.d_slots, t.slots.data(), t.slots.size() * sizeof(PoseSlot), 0}};
+  Layout l;
+  for (Part& p : parts) p.off = l.add(std::max<size_t>(p.bytes, 4));
+  const size_t tables = l.end, total = std::max<size_t>(t.slots.size(), 1);
+  const size_t keys = l.add(total * sizeof(unsigned long long));
+  const size_t meta = l.add(total * sizeof(RotMeta));
+  if (t.h_up_busy) hip_check(hipStreamSynchronize(ctx.stream), "upload sync");
+  t.h_up_busy = false;
+  if (tables > t.h_up_cap) {
+    if (t.h_up) (void)hipHostFree(t.h_up);
+    t.h_up = nullptr;
+    t.h_up_cap = 0;
+    hip_check(hipHostMalloc(&t.h_up, tables), "hipHostMalloc");
+    t.h_up_cap = tables;
   }
-  const size_t total = std::max<size_t>(t.slots.size(), 1);
-  t.d_keys.ensure(total * sizeof(unsigned long long));
-  t.d_meta.ensure(total * sizeof(RotMeta));
+  t.d_all.ensure(l.end);
+  char* d = t.d_all.as<char>();
+  char* h = static_cast<char*>(t.h_up);
+  for (const Part& p : parts) {
+    p.dst->p = d + p.off;
+    if (p.bytes) std::memcpy(h + p.off, p.src, p.bytes);
+  }
+  hip_check(hipMemcpyAsync(d, h, tables, hipMemcpyHostToDevice, ctx.stream), "tables H2D");
+  t.h_up_busy = true;
+  t.d_keys.p = d + keys;
+  t.d_meta.p = d + meta;
+  t.res_meta = meta - keys;
+  t.res_bytes = t.res_meta + total * sizeof(RotMeta);
 }
 
 }  // namespace
@@ -1065,13 +1147,12 @@ void prepare_search(Context& ctx, const Protein& prot, const std::vector<Job>& j
   std::lock_guard<std::mutex> lock(ctx.mu);
   hip_check(hipSetDevice(ctx.device), "hipSetDevice");
   upload_tables(ctx, t);
-  hip_check(hipStreamSynchronize(ctx.stream), "prepare sync");
 }
 
 namespace {
 
 // Enqueues t's launch sequence and the copies of its keys and per-pose
-// metadata to host staging (t's own when t.own_staging, else the context's);
+// metadata to t's pinned staging;
 // context lock held.
 void enqueue_search(Context& ctx, Prepared& t, Engine engine, bool use_graph, EventTimer& timer,
                     hipEvent_t start = nullptr) {
@@ -1134,39 +1215,46 @@ void enqueue_search(Context& ctx, Prepared& t, Engine engine, bool use_graph, Ev
       enqueue_fused(ctx, prot, t, chunk, tu, timer);
     }
   }
-  void* hk = ctx.h_keys;
-  void* hm = ctx.h_meta;
-  if (t.own_staging) {
-    if (total > t.h_cap) {
-      if (t.h_keys) (void)hipHostFree(t.h_keys);
-      if (t.h_meta) (void)hipHostFree(t.h_meta);
-      t.h_keys = t.h_meta = nullptr;
-      t.h_cap = 0;
-      hip_check(hipHostMalloc(&t.h_keys, total * sizeof(unsigned long long)), "hipHostMalloc");
-      hip_check(hipHostMalloc(&t.h_meta, total * sizeof(RotMeta)), "hipHostMalloc");
-      t.h_cap = total;
-    }
-    hk = t.h_keys;
-    hm = t.h_meta;
-  } else {
-    ctx.ensure_host(total);
-    hk = ctx.h_keys;
-    hm = ctx.h_meta;
+  if (t.res_bytes > t.h_res_cap) {
+    if (t.h_res) (void)hipHostFree(t.h_res);
+    t.h_res = nullptr;
+    t.h_res_cap = 0;
+    hip_check(hipHostMalloc(&t.h_res, t.res_bytes), "hipHostMalloc");
+    t.h_res_cap = t.res_bytes;
   }
-  hip_check(hipMemcpyAsync(hk, t.d_keys.p, total * sizeof(unsigned long long), hipMemcpyDeviceToHost, ctx.stream),
-            "keys D2H");
-  hip_check(hipMemcpyAsync(hm, t.d_meta.p, total * sizeof(RotMeta), hipMemcpyDeviceToHost, ctx.stream), "meta D2H");
+  hip_check(hipMemcpyAsync(t.h_res, t.d_keys.p, t.res_bytes, hipMemcpyDeviceToHost, ctx.stream), "results D2H");
 }
 
-// Per-pose results of t from host staging (keys, metadata).
-void decode_results(Prepared& t, const void* hkeys, const void* hmeta) {
-  const Protein& prot = *t.prot;
-  const unsigned long long* keys = static_cast<const unsigned long long*>(hkeys);
-  const RotMeta* meta = static_cast<const RotMeta*>(hmeta);
-  const int N = prot.N;
+// Poses first .. first + n - 1 of t from its host staging; index, mincoor, box
+// and win optional ([n][3] each).
+void decode_poses(const Prepared& t, size_t first, size_t n, float* energy, int* index, float* mincoor, int* box,
+                  int* win) {
+  const unsigned long long* keys = static_cast<const unsigned long long*>(t.h_res) + first;
+  const RotMeta* meta =
+      reinterpret_cast<const RotMeta*>(static_cast<const char*>(t.h_res) + t.res_meta) + first;
+  const unsigned N = (unsigned)t.prot->N;
+  for (size_t i = 0; i < n; ++i) {
+    const unsigned long long k = keys[i];
+    const RotMeta& m = meta[i];
+    const bool found = k != ~0ull && m.valid;
+    energy[i] = found ? key_energy(k) : std::numeric_limits<float>::infinity();
+    if (index) {
+      const unsigned lin = key_index(k);
+      index[i * 3 + 0] = found ? (int)(lin / (N * N)) : -1;
+      index[i * 3 + 1] = found ? (int)((lin / N) % N) : -1;
+      index[i * 3 + 2] = found ? (int)(lin % N) : -1;
+    }
+    for (int c = 0; c < 3; ++c) {
+      if (mincoor) mincoor[i * 3 + c] = m.minc[c];
+      if (box) box[i * 3 + c] = m.box[c];
+      if (win) win[i * 3 + c] = m.win[c];
+    }
+  }
+}
+
+void decode_results(Prepared& t) {
   t.results.assign(t.job_first.size(), PoseResults());
   for (size_t j = 0; j < t.job_first.size(); ++j) {
-    const size_t first = t.job_first[j];
     const size_t n = t.job_n[j];
     PoseResults& r = t.results[j];
     r.energy.resize(n);
@@ -1174,26 +1262,19 @@ void decode_results(Prepared& t, const void* hkeys, const void* hmeta) {
     r.mincoor.resize(n * 3);
     r.box.resize(n * 3);
     r.win.resize(n * 3);
-    for (size_t i = 0; i < n; ++i) {
-      const unsigned long long k = keys[first + i];
-      const RotMeta& m = meta[first + i];
-      if (k == ~0ull || !m.valid) {
-        r.energy[i] = std::numeric_limits<float>::infinity();
-        r.index[i * 3 + 0] = r.index[i * 3 + 1] = r.index[i * 3 + 2] = -1;
-      } else {
-        const unsigned lin = key_index(k);
-        r.energy[i] = key_energy(k);
-        r.index[i * 3 + 0] = (int)(lin / (unsigned)(N * N));
-        r.index[i * 3 + 1] = (int)((lin / (unsigned)N) % (unsigned)N);
-        r.index[i * 3 + 2] = (int)(lin % (unsigned)N);
-      }
-      for (int k3 = 0; k3 < 3; ++k3) {
-        r.mincoor[i * 3 + k3] = m.minc[k3];
-        r.box[i * 3 + k3] = m.box[k3];
-        r.win[i * 3 + k3] = m.win[k3];
-      }
-    }
+    decode_poses(t, t.job_first[j], n, r.energy.data(), r.index.data(), r.mincoor.data(), r.box.data(), r.win.data());
   }
+}
+
+// Runs t's launch sequence to its end (context lock held).
+void run_prepared(Context& ctx, Prepared& t, Engine engine, bool use_graph) {
+  EventTimer timer(ctx);
+  t.own_staging = false;
+  enqueue_search(ctx, t, engine, use_graph, timer);
+  hip_check(hipStreamSynchronize(ctx.stream), "search sync");
+  t.h_up_busy = false;
+  t.ran = true;
+  timer.collect();
 }
 
 }  // namespace
@@ -1204,13 +1285,8 @@ void execute_search(Context& ctx, Prepared& t, Engine engine, bool use_graph) {
   if (!t.prot) throw Error(kErrInvalid, "search not prepared");
   t.results.assign(t.job_first.size(), PoseResults());
   if (t.slots.empty()) return;
-  EventTimer timer(ctx);
-  t.own_staging = false;
-  enqueue_search(ctx, t, engine, use_graph, timer);
-  hip_check(hipStreamSynchronize(ctx.stream), "search sync");
-  timer.collect();
-  // Decode while the pinned staging is ours (context lock held).
-  decode_results(t, ctx.h_keys, ctx.h_meta);
+  run_prepared(ctx, t, engine, use_graph);
+  decode_results(t);
 }
 
 void submit_search(Context& ctx, Prepared& t) {
@@ -1243,7 +1319,8 @@ void finish_search(Context& ctx, Prepared& t) {
   if (!t.done) throw Error(kErrInvalid, "search not submitted");
   hip_check(hipEventSynchronize(t.done), "search wait");
   t.results.assign(t.job_first.size(), PoseResults());
-  if (!t.slots.empty()) decode_results(t, t.h_keys, t.h_meta);
+  t.h_up_busy = false;
+  if (!t.slots.empty()) decode_results(t);
 }
 
 float search_gpu_ms(Prepared& t) {
@@ -1252,12 +1329,42 @@ float search_gpu_ms(Prepared& t) {
   return ms;
 }
 
-void run_search(Context& ctx, const Protein& prot, const std::vector<Job>& jobs, Engine engine,
-                std::vector<PoseResults>& out) {
-  Prepared t;
-  prepare_search(ctx, prot, jobs, t);
-  execute_search(ctx, t, engine, false);
-  out = std::move(t.results);
+void run_search(Context& ctx, const Protein& prot, const Job& job, Engine engine, float* energy, int* index,
+                float* mincoor) {
+  std::unique_ptr<Prepared> t;
+  {
+    std::lock_guard<std::mutex> lock(ctx.idle_mu);
+    if (!ctx.idle.empty()) {
+      t = std::move(ctx.idle.back());
+      ctx.idle.pop_back();
+    }
+  }
+  if (!t) t = std::make_unique<Prepared>();
+  {
+    // a call that fails leaves nothing queued that reads t's staging
+    struct Drain {
+      Context& ctx;
+      Prepared& t;
+      ~Drain() {
+        if (t.h_up_busy) (void)hipStreamSynchronize(ctx.stream);
+        t.h_up_busy = false;
+      }
+    } drain{ctx, *t};
+    build_search(prot, {job}, *t);
+    std::lock_guard<std::mutex> lock(ctx.mu);
+    hip_check(hipSetDevice(ctx.device), "hipSetDevice");
+    upload_tables(ctx, *t);
+    if (!t->slots.empty()) {
+      run_prepared(ctx, *t, engine, false);
+      decode_poses(*t, 0, t->slots.size(), energy, index, mincoor, nullptr, nullptr);
+    }
+  }
+  t->prot = nullptr;
+  if (t->d_all.cap <= Context::kIdleBytes && t->h_up_cap <= Context::kIdleBytes &&
+      t->h_res_cap <= Context::kIdleBytes) {
+    std::lock_guard<std::mutex> lock(ctx.idle_mu);
+    if (ctx.idle.size() < Context::kIdleSearches) ctx.idle.push_back(std::move(t));
+  }
 }
 
 namespace {
@@ -1272,26 +1379,42 @@ void atom_channels(const Protein& prot, const Ligand& lig, std::vector<int>& pch
   (void)prot;
 }
 
-struct PoseScratch {
-  DevBuf coords, pch, wv, wq, energy, grad, inside;
+// Poses whose coordinates (and gradients) go through the pinned arena at a
+// time, and the parts of that arena: the ligand's channels and weights, then
+// the poses' coordinates and results.  The kernels read and write them in
+// place over the host link.
+struct PoseStage {
+  int per = 0;  // poses per piece
+  int *pch = nullptr, *inside = nullptr;
+  float *wv = nullptr, *wq = nullptr;
+  double *x = nullptr, *g = nullptr, *e = nullptr;
 };
+constexpr size_t kPoseStageBytes = 32ull << 20;
 
-void stage_pose_inputs(Context& ctx, const Protein& prot, const Ligand& lig, int npose, const double* coords,
-                       PoseScratch& w) {
+PoseStage stage_poses(CallScratch& scratch, const Protein& prot, const Ligand& lig, int npose, bool grad) {
+  const size_t na = (size_t)lig.natom, pose = na * 3 * sizeof(double);
+  PoseStage s;
+  s.per = (int)std::max<size_t>(1, std::min<size_t>((size_t)npose, kPoseStageBytes / ((grad ? 2 : 1) * pose + 16)));
+  Layout l;
+  const size_t o_pch = l.add(na * sizeof(int)), o_wv = l.add(na * sizeof(float)), o_wq = l.add(na * sizeof(float));
+  const size_t o_e = l.add(s.per * sizeof(double)), o_in = l.add(s.per * sizeof(int));
+  const size_t o_x = l.add(s.per * pose), o_g = grad ? l.add(s.per * pose) : 0;
+  char* h = scratch.host(l.end);
+  s.pch = reinterpret_cast<int*>(h + o_pch);
+  s.wv = reinterpret_cast<float*>(h + o_wv);
+  s.wq = reinterpret_cast<float*>(h + o_wq);
+  s.e = reinterpret_cast<double*>(h + o_e);
+  s.inside = reinterpret_cast<int*>(h + o_in);
+  s.x = reinterpret_cast<double*>(h + o_x);
+  if (grad) s.g = reinterpret_cast<double*>(h + o_g);
   std::vector<int> pch;
   atom_channels(prot, lig, pch);
-  std::vector<float> wv(lig.natom), wq(lig.natom);
   for (int a = 0; a < lig.natom; ++a) {
-    wv[a] = std::sqrt(lig.eps[a]);
-    wq[a] = lig.charge[a];
+    s.pch[a] = pch[a];
+    s.wv[a] = std::sqrt(lig.eps[a]);
+    s.wq[a] = lig.charge[a];
   }
-  upload(ctx, w.pch, pch);
-  upload(ctx, w.wv, wv);
-  upload(ctx, w.wq, wq);
-  const size_t n = (size_t)npose * lig.natom * 3;
-  w.coords.ensure(std::max<size_t>(n, 1) * sizeof(double));
-  if (n) hip_check(hipMemcpyAsync(w.coords.p, coords, n * sizeof(double), hipMemcpyHostToDevice, ctx.stream), "coords");
-  w.energy.ensure(std::max(npose, 1) * sizeof(double));
+  return s;
 }
 
 }  // namespace
@@ -1301,25 +1424,21 @@ void rescore_poses(Context& ctx, const Protein& prot, const Ligand& lig, int npo
   std::lock_guard<std::mutex> lock(ctx.mu);
   hip_check(hipSetDevice(ctx.device), "hipSetDevice");
   if (npose <= 0) return;
-  PoseScratch w;
-  stage_pose_inputs(ctx, prot, lig, npose, coords, w);
-  const size_t n = (size_t)npose * lig.natom * 3;
-  if (grad) w.grad.ensure(n * sizeof(double));
-  if (inside) w.inside.ensure((size_t)npose * sizeof(int));
+  CallScratch scratch(ctx);
+  const PoseStage w = stage_poses(scratch, prot, lig, npose, grad != nullptr);
   const double gmin[3] = {prot.grid_min(0), prot.grid_min(1), prot.grid_min(2)};
-  hip_check(launch_rescore(ctx.stream, npose, lig.natom, w.coords.as<double>(), w.pch.as<int>(), w.wv.as<float>(),
-                           w.wq.as<float>(), prot.grid.as<float>(), prot.N, prot.nch - 1, gmin, (double)prot.h,
-                           w.energy.as<double>(), grad ? w.grad.as<double>() : nullptr,
-                           inside ? w.inside.as<int>() : nullptr),
-            "rescore");
-  hip_check(hipMemcpyAsync(energy, w.energy.p, (size_t)npose * sizeof(double), hipMemcpyDeviceToHost, ctx.stream),
-            "energy D2H");
-  if (grad)
-    hip_check(hipMemcpyAsync(grad, w.grad.p, n * sizeof(double), hipMemcpyDeviceToHost, ctx.stream), "grad D2H");
-  if (inside)
-    hip_check(hipMemcpyAsync(inside, w.inside.p, (size_t)npose * sizeof(int), hipMemcpyDeviceToHost, ctx.stream),
-              "inside D2H");
-  hip_check(hipStreamSynchronize(ctx.stream), "rescore sync");
+  const size_t per = (size_t)lig.natom * 3;
+  for (int p0 = 0; p0 < npose; p0 += w.per) {
+    const int n = std::min(w.per, npose - p0);
+    std::memcpy(w.x, coords + p0 * per, n * per * sizeof(double));
+    hip_check(launch_rescore(ctx.stream, n, lig.natom, w.x, w.pch, w.wv, w.wq, prot.grid.as<float>(), prot.N,
+                             prot.nch - 1, gmin, (double)prot.h, w.e, w.g, w.inside),
+              "rescore");
+    hip_check(hipStreamSynchronize(ctx.stream), "rescore sync");
+    std::memcpy(energy + p0, w.e, n * sizeof(double));
+    if (grad) std::memcpy(grad + p0 * per, w.g, n * per * sizeof(double));
+    if (inside) std::memcpy(inside + p0, w.inside, n * sizeof(int));
+  }
 }
 
 void refine_poses(Context& ctx, const Protein& prot, const Ligand& lig, int npose, double* coords, int steps,
@@ -1327,18 +1446,20 @@ void refine_poses(Context& ctx, const Protein& prot, const Ligand& lig, int npos
   std::lock_guard<std::mutex> lock(ctx.mu);
   hip_check(hipSetDevice(ctx.device), "hipSetDevice");
   if (npose <= 0) return;
-  PoseScratch w;
-  stage_pose_inputs(ctx, prot, lig, npose, coords, w);
-  const size_t n = (size_t)npose * lig.natom * 3;
+  CallScratch scratch(ctx);
+  const PoseStage w = stage_poses(scratch, prot, lig, npose, false);
   const double gmin[3] = {prot.grid_min(0), prot.grid_min(1), prot.grid_min(2)};
-  hip_check(launch_refine(ctx.stream, npose, lig.natom, w.coords.as<double>(), w.pch.as<int>(), w.wv.as<float>(),
-                          w.wq.as<float>(), prot.grid.as<float>(), prot.N, prot.nch - 1, gmin, (double)prot.h, steps,
-                          penalty, w.energy.as<double>()),
-            "refine");
-  hip_check(hipMemcpyAsync(coords, w.coords.p, n * sizeof(double), hipMemcpyDeviceToHost, ctx.stream), "coords D2H");
-  hip_check(hipMemcpyAsync(energy, w.energy.p, (size_t)npose * sizeof(double), hipMemcpyDeviceToHost, ctx.stream),
-            "energy D2H");
-  hip_check(hipStreamSynchronize(ctx.stream), "refine sync");
+  const size_t per = (size_t)lig.natom * 3;
+  for (int p0 = 0; p0 < npose; p0 += w.per) {
+    const int n = std::min(w.per, npose - p0);
+    std::memcpy(w.x, coords + p0 * per, n * per * sizeof(double));
+    hip_check(launch_refine(ctx.stream, n, lig.natom, w.x, w.pch, w.wv, w.wq, prot.grid.as<float>(), prot.N,
+                            prot.nch - 1, gmin, (double)prot.h, steps, penalty, w.e),
+              "refine");
+    hip_check(hipStreamSynchronize(ctx.stream), "refine sync");
+    std::memcpy(coords + p0 * per, w.x, n * per * sizeof(double));
+    std::memcpy(energy + p0, w.e, n * sizeof(double));
+  }
 }
 
 int generate_conformers(Context& ctx, int natom, const double* coords, int nrotor, const int* rotors,
@@ -1351,59 +1472,60 @@ int generate_conformers(Context& ctx, int natom, const double* coords, int nroto
     for (int k = 0; k < 4; ++k)
       if (rotors[r * 4 + k] < 0 || rotors[r * 4 + k] >= natom) throw Error(kErrInvalid, "rotor atom out of range");
   const size_t per = (size_t)natom * 3;
-  std::vector<double> x(coords, coords + per);
-  std::vector<int> rot(rotors, rotors + (size_t)nrotor * 4);
   const int rw = (nrotor + 63) / 64, ew = (natom + 63) / 64;
-  std::vector<unsigned long long> mv((size_t)rw * natom, 0ull), ex((size_t)natom * ew, 0ull);
-  for (int r = 0; r < nrotor; ++r)
-    for (int a = 0; a < natom; ++a)
-      if (moving[(size_t)r * natom + a]) mv[(size_t)(r / 64) * natom + a] |= 1ull << (r % 64);
-  for (int a = 0; a < natom; ++a)
-    for (int b = 0; b < natom; ++b)
-      if (exclude[(size_t)a * natom + b]) ex[(size_t)a * ew + b / 64] |= 1ull << (b % 64);
-  DevBuf d_x, d_rot, d_mv, d_ex, d_out, d_ok, d_list, d_kept, d_trial;
-  upload(ctx, d_x, x);
-  upload(ctx, d_rot, rot);
-  upload(ctx, d_mv, mv);
-  upload(ctx, d_ex, ex);
   // Trials run a set at a time and stop once enough have passed: the kept
   // ones are the first max_keep in trial order, so later trials cannot
   // matter.  A first set of 4 096 (four wavefronts per SIMD) takes hardly
   // longer than one of a few; the next sets follow the share that passed.
   int kept = 0, done = 0;
   int set = std::min(ntrial, std::max(4096, max_keep));
+  // no later set is larger than this
+  const size_t cap = (size_t)std::min<long long>(ntrial, std::max(1 << 16, set));
+  const size_t keep = std::min<size_t>(max_keep, cap);
+  CallScratch scratch(ctx);
+  Layout in, l;
+  const size_t o_x = in.add(per * sizeof(double)), o_rot = in.add((size_t)nrotor * 4 * sizeof(int));
+  const size_t o_mv = in.add((size_t)rw * natom * 8), o_ex = in.add((size_t)natom * ew * 8);
+  l.add(in.end);
+  const size_t o_ok = l.add(cap * sizeof(int)), o_list = l.add(keep * sizeof(int));
+  const size_t o_count = l.add(sizeof(int)), o_trial = l.add(keep * sizeof(int));
+  const size_t o_kept = l.add(keep * per * sizeof(double)), o_all = l.add(cap * per * sizeof(double));
+  char* d = scratch.dev(l.end);
+  char* h = scratch.host(in.end);
+  std::memcpy(h + o_x, coords, per * sizeof(double));
+  if (nrotor) std::memcpy(h + o_rot, rotors, (size_t)nrotor * 4 * sizeof(int));
+  unsigned long long* mv = reinterpret_cast<unsigned long long*>(h + o_mv);
+  unsigned long long* ex = reinterpret_cast<unsigned long long*>(h + o_ex);
+  std::fill(mv, mv + (size_t)rw * natom, 0ull);
+  std::fill(ex, ex + (size_t)natom * ew, 0ull);
+  for (int r = 0; r < nrotor; ++r)
+    for (int a = 0; a < natom; ++a)
+      if (moving[(size_t)r * natom + a]) mv[(size_t)(r / 64) * natom + a] |= 1ull << (r % 64);
+  for (int a = 0; a < natom; ++a)
+    for (int b = 0; b < natom; ++b)
+      if (exclude[(size_t)a * natom + b]) ex[(size_t)a * ew + b / 64] |= 1ull << (b % 64);
+  hip_check(hipMemcpyAsync(d, h, in.end, hipMemcpyHostToDevice, ctx.stream), "conformer inputs H2D");
   while (done < ntrial && kept < max_keep) {
     const int need = std::min(max_keep - kept, set);
-    d_out.ensure((size_t)set * per * sizeof(double));
-    d_ok.ensure((size_t)set * sizeof(int));
-    d_list.ensure((size_t)(need + 1) * sizeof(int));
-    d_kept.ensure((size_t)need * per * sizeof(double));
-    d_trial.ensure((size_t)need * sizeof(int));
-    int* d_count = d_list.as<int>() + need;
-    hip_check(launch_conformers(ctx.stream, natom, d_x.as<double>(), nrotor, d_rot.as<int>(),
-                                d_mv.as<unsigned long long>(), d_ex.as<unsigned long long>(), done, set, seed,
-                                clash_dist, d_out.as<double>(), d_ok.as<int>()),
+    hip_check(launch_conformers(ctx.stream, natom, reinterpret_cast<double*>(d + o_x), nrotor,
+                                reinterpret_cast<int*>(d + o_rot), reinterpret_cast<unsigned long long*>(d + o_mv),
+                                reinterpret_cast<unsigned long long*>(d + o_ex), done, set, seed, clash_dist,
+                                reinterpret_cast<double*>(d + o_all), reinterpret_cast<int*>(d + o_ok)),
               "conformers");
-    hip_check(launch_keep_conformers(ctx.stream, natom, done, set, d_ok.as<int>(), d_out.as<double>(), need,
-                                     d_list.as<int>(), d_count, d_kept.as<double>(), d_trial.as<int>()),
+    hip_check(launch_keep_conformers(ctx.stream, natom, done, set, reinterpret_cast<int*>(d + o_ok),
+                                     reinterpret_cast<double*>(d + o_all), need, reinterpret_cast<int*>(d + o_list),
+                                     reinterpret_cast<int*>(d + o_count), reinterpret_cast<double*>(d + o_kept),
+                                     reinterpret_cast<int*>(d + o_trial)),
               "conformers kept");
     int n = 0;
-    hip_check(hipMemcpyAsync(&n, d_count, sizeof(int), hipMemcpyDeviceToHost, ctx.stream), "count D2H");
-    hip_check(hipStreamSynchronize(ctx.stream), "conformers sync");
-    if (n > 0) {
-      hip_check(hipMemcpyAsync(out + (size_t)kept * per, d_kept.p, (size_t)n * per * sizeof(double),
-                               hipMemcpyDeviceToHost, ctx.stream),
-                "conformers D2H");
-      if (trial_index)
-        hip_check(hipMemcpyAsync(trial_index + kept, d_trial.p, (size_t)n * sizeof(int), hipMemcpyDeviceToHost,
-                                 ctx.stream),
-                  "trials D2H");
-      hip_check(hipStreamSynchronize(ctx.stream), "conformers sync");
-    }
+    scratch.out(&n, d + o_count, sizeof(int));
+    scratch.out(out + (size_t)kept * per, d + o_kept, (size_t)n * per * sizeof(double));
+    if (trial_index) scratch.out(trial_index + kept, d + o_trial, (size_t)n * sizeof(int));
     kept += n;
     done += set;
     const double pass = (double)std::max(kept, 1) / done;
-    set = (int)std::min<double>(ntrial - done, std::max(4096.0, 1.25 * (max_keep - kept) / pass));
+    set = (int)std::min<double>(std::min<double>(ntrial - done, (double)cap),
+                                std::max(4096.0, 1.25 * (max_keep - kept) / pass));
   }
   return kept;
 }

@@ -48,7 +48,52 @@ struct DevBuf {
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
+// Part of a device allocation.
+struct DevView {
+  void* p = nullptr;
+  template <class T> T* as() const { return static_cast<T*>(p); }
+};
+
 struct Context;
+
+// One call's use of its context's scratch memory (the context lock held for
+// the object's life): a device arena and a pinned host arena that grow to what
+// a call needs and stay with the context for the next, up to kKeepDev and
+// kKeepHost bytes; a call that needed more gives the excess back when it ends.
+// A call that ends by an exception waits for the stream first, so nothing
+// queued still reads or writes the arenas.
+class CallScratch {
+ public:
+  static constexpr size_t kKeepDev = 128ull << 20, kKeepHost = 64ull << 20;
+  explicit CallScratch(Context& c);
+  ~CallScratch();
+  CallScratch(const CallScratch&) = delete;
+  CallScratch& operator=(const CallScratch&) = delete;
+  // The arena's start, at least `bytes` long; once per call each.
+  char* dev(size_t bytes);
+  char* host(size_t bytes);
+  // Host memory of the caller to device memory and back through pinned
+  // slots, the host's copy of one piece beside the transfer of another
+  // (a copy straight from or to pageable memory stages the same bytes with no
+  // overlap).  in() leaves the last transfers queued on the context stream;
+  // out() returns when dst is written.  Both use the host arena.
+  void in(void* dev_dst, const void* src, size_t bytes);
+  void out(void* dst, const void* dev_src, size_t bytes);
+
+ private:
+  Context& ctx_;
+  int exceptions_;
+};
+
+// Offsets of the 256-byte aligned parts of an arena.
+struct Layout {
+  size_t end = 0;
+  size_t add(size_t bytes) {
+    const size_t o = end;
+    end += (bytes + 255) & ~(size_t)255;
+    return o;
+  }
+};
 
 // Resident protein: potential grids and their forward spectra, all channels,
 // FP32, [channel][X][Y][Z] and [channel][X][Y][Z/2+1] (NoMini:177-199).
@@ -60,11 +105,12 @@ struct Protein {
   float mid[3] = {0, 0, 0};
   float len[3] = {0, 0, 0};
   std::vector<float> radii;  // nch - 1 probe radii
-  DevBuf grid;               // float [nch][G]
-  DevBuf spec;               // float2 [nch][H]
-  DevBuf spec_lb;            // the same spectra in the fused engine's line-blocked layout
-  DevBuf spec_kz;            // and in the column form's kz-plane layout (grid edge 64 only)
-  DevBuf spec_mf;            // and in the atom form's matrix-core layout (grid edge 64 only)
+  DevBuf all;                // one allocation: the grids and every copy of the spectra
+  DevView grid;              // float [nch][G]
+  DevView spec;              // float2 [nch][H]
+  DevView spec_lb;           // the same spectra in the fused engine's line-blocked layout
+  DevView spec_kz;           // and in the column form's kz-plane layout (grid edge 64 only)
+  DevView spec_mf;           // and in the atom form's matrix-core layout (grid edges 64, 96 and 128)
   size_t G() const { return (size_t)N * N * N; }
   size_t H() const { return (size_t)N * N * (N / 2 + 1); }
   // gridMin = mid - len / 2 evaluated in float, then widened (NoMini:149-151).
@@ -137,7 +183,13 @@ struct Prepared {
   std::vector<size_t> job_first, job_n;
   int astride = 0, cmax = 0, boxmax = 2, max_chan_atoms = 1;
   int dummy_lig = 0;
-  DevBuf d_ligs, d_chan, d_pad, d_wv, d_wq, d_coords, d_slots, d_keys, d_meta;
+  // one device allocation: the tables (uploaded as one piece), then the keys
+  // and the per-pose metadata (copied back as one piece, `res_bytes` from
+  // d_keys on, the metadata res_meta bytes in)
+  DevBuf d_all;
+  DevView d_ligs, d_chan, d_pad, d_wv, d_wq, d_coords, d_slots, d_keys, d_meta;
+  size_t res_bytes = 0, res_meta = 0;
+  bool ran = false;  // executed since it was built
   hipGraphExec_t graph = nullptr;
   uint64_t graph_gen = 0;
   size_t graph_chunk = 0;
@@ -151,9 +203,9 @@ struct Prepared {
   bool own_staging = false;
   void* h_up = nullptr;  // pinned staging of the tables' upload
   size_t h_up_cap = 0;
-  void* h_keys = nullptr;
-  void* h_meta = nullptr;
-  size_t h_cap = 0;
+  bool h_up_busy = false;  // its last upload may still be queued
+  void* h_res = nullptr;   // own pinned staging of the results
+  size_t h_res_cap = 0;
   hipEvent_t start = nullptr, done = nullptr;
   Prepared() = default;
   Prepared(const Prepared&) = delete;
@@ -218,15 +270,21 @@ struct Context {
   // the reference dataflow's batch arrays
   DevBuf d_L, d_Lhat, d_S, d_E;
   uint64_t ws_generation = 1;
-  // pinned host staging
-  void* h_keys = nullptr;
-  void* h_meta = nullptr;
-  size_t h_cap = 0;
+  // scratch of the synchronous calls (CallScratch)
+  DevBuf call_dev;
+  void* call_host = nullptr;
+  size_t call_host_cap = 0;
+  std::vector<hipEvent_t> call_events;
+  // Tables of finished cdk_search calls, kept for the next ones: at most
+  // kIdleSearches of at most kIdleBytes each.  Every call takes one for
+  // itself, so calls of several threads never share one.
+  static constexpr size_t kIdleSearches = 2, kIdleBytes = 64ull << 20;
+  std::mutex idle_mu;
+  std::vector<std::unique_ptr<Prepared>> idle;
 
   explicit Context(int dev);
   ~Context();
   const float2* twiddle(int N);
-  void ensure_host(size_t nslots);
 };
 
 void protein_upload(Protein& p, int nch, int N, float h, const float* mid, const float* len, const float* radii,
@@ -260,9 +318,10 @@ void submit_search(Context& ctx, Prepared& t);
 void finish_search(Context& ctx, Prepared& t);
 // GPU milliseconds of t's last submitted sequence (after finish_search).
 float search_gpu_ms(Prepared& t);
-// prepare + execute without a graph.
-void run_search(Context& ctx, const Protein& prot, const std::vector<Job>& jobs, Engine engine,
-                std::vector<PoseResults>& out);
+// prepare + execute without a graph, one job; results straight to the caller's
+// arrays (index and mincoor optional).
+void run_search(Context& ctx, const Protein& prot, const Job& job, Engine engine, float* energy, int* index,
+                float* mincoor);
 
 // Grid score of explicit poses (FP64 trilinear, see rescore.hip): coords
 // [npose][natom][3] in A; energy [npose]; grad [npose][natom][3] and inside

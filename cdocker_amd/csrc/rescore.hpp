@@ -4,10 +4,11 @@
 
 namespace cdk {
 
-// coords [npose][natom][3] (A); pch[a] = protein probe channel of atom a
+// coords [npose][natom][3] (A), 16-byte aligned; pch[a] = protein probe channel of atom a
 // (-1: none), ech = elec channel; wv = sqrt(eps), wq = charge; gmin = grid
 // origin.  energy [npose]; grad [npose][natom][3] (optional, kcal/mol/A);
 // inside [npose] = atoms on the grid (optional).
+// Every array but grid may be pinned host memory.
 hipError_t launch_rescore(hipStream_t st, int npose, int natom, const double* coords, const int* pch,
                           const float* wv, const float* wq, const float* grid, int N, int ech, const double* gmin,
                           double h, double* energy, double* grad, int* inside);
