@@ -174,13 +174,91 @@ __device__ __forceinline__ void reg_twiddles(const float2* __restrict__ tw, int 
   for (int k1 = 0; k1 < RegShape<N>::V; ++k1) twl[k1] = tw[n2 * k1];
 }
 
-// One transform of the wavefront's lines.  `lds` is the wavefront's slice of
-// RegShape<N>::SLICE float2.  ln = line within the wavefront, n2 = lane
+// a's upper and b's lower halves change places, in blocks of B lanes: of
+// every 2 B lanes, the upper B of a and the lower B of b.
+template <int B>
+__device__ __forceinline__ void lane_swap(float& a, float& b) {
+  const int ia = __float_as_int(a), ib = __float_as_int(b);
+  if constexpr (B == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(ia, ib, false, false);
+    a = __int_as_float(r[0]);
+    b = __int_as_float(r[1]);
+  } else if constexpr (B == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(ia, ib, false, false);
+    a = __int_as_float(r[0]);
+    b = __int_as_float(r[1]);
+  } else {
+    static_assert(B == 8, "halves of a row of 16");
+    // row_ror:8 into the upper (lower) 8 lanes of each row
+    a = __int_as_float(__builtin_amdgcn_update_dpp(ia, ib, 0x128, 0xf, 0xc, false));
+    b = __int_as_float(__builtin_amdgcn_update_dpp(ib, ia, 0x128, 0xf, 0x3, false));
+  }
+}
+template <int B>
+__device__ __forceinline__ void lane_swap(float2& a, float2& b) {
+  lane_swap<B>(a.x, b.x);
+  lane_swap<B>(a.y, b.y);
+}
+
+// u[r] on lane group m (lane / (64 / L) = m) -> u[m] on lane group r.
+template <int L>
+__device__ __forceinline__ void lane_transpose(float2* u) {
+  static_assert(L == 4 || L == 8, "4 or 8 lane groups");
+#pragma unroll
+  for (int i = 0; i < L / 2; ++i) lane_swap<32>(u[i], u[i + L / 2]);
+#pragma unroll
+  for (int h = 0; h < L; h += L / 2)
+#pragma unroll
+    for (int i = 0; i < L / 4; ++i) lane_swap<16>(u[h + i], u[h + i + L / 4]);
+  if constexpr (L == 8) {
+#pragma unroll
+    for (int i = 0; i < L; i += 2) lane_swap<8>(u[i], u[i + 1]);
+  }
+}
+
+// One transform of the wavefront's lines (all lanes active): lane n2 * LPW +
+// ln holds value j of line ln at n2 + L j, before and after.  n2 = lane
 // within the line.
+// HALF: inputs x[n] with n >= N/2 are zero (registers V/2.. are not read).
+template <int N, int S, bool HALF = false>
+__device__ __forceinline__ void lane_fft(float2* v, const float2* twl) {
+  constexpr int L = RegShape<N>::L, V = RegShape<N>::V;
+  if constexpr (HALF)
+    RegDFTHalf<V, S>::run(v);
+  else
+    RegDFT<V, S>::run(v);
+#pragma unroll
+  for (int k1 = 1; k1 < V; ++k1) {
+    float2 w = twl[k1];
+    if (S > 0) w.y = -w.y;
+    v[k1] = c_mul(v[k1], w);
+  }
+  float2 o[V];
+#pragma unroll
+  for (int q = 0; q < V / L; ++q) {
+    float2* u = v + q * L;
+    lane_transpose<L>(u);
+    SmallDFT<L, S>::run(u);
+#pragma unroll
+    for (int k2 = 0; k2 < L; ++k2) o[q + (V / L) * k2] = u[k2];
+  }
+#pragma unroll
+  for (int j = 0; j < V; ++j) v[j] = o[j];
+}
+
+// One transform of the wavefront's lines (all lanes active).  With four lanes
+// per line the lanes trade values directly (lane_fft); with eight (three
+// exchanges instead of two, the last one two moves) through `lds`, the
+// wavefront's slice of RegShape<N>::SLICE float2.  ln = line within the
+// wavefront, n2 = lane within the line.
 // HALF: inputs x[n] with n >= N/2 are zero (registers V/2.. are not read).
 template <int N, int S, bool HALF = false>
 __device__ __forceinline__ void reg_fft(float2* v, const float2* twl, float2* lds, int ln, int n2) {
   constexpr int L = RegShape<N>::L, V = RegShape<N>::V;
+  if constexpr (L == 4) {
+    lane_fft<N, S, HALF>(v, twl);
+    return;
+  }
   if constexpr (HALF)
     RegDFTHalf<V, S>::run(v);
   else

@@ -2662,7 +2662,15 @@ __global__ __launch_bounds__(128 * AtomTab::NP) __attribute__((amdgpu_waves_per_
 // one complex line (two-for-one, imaginary parts of the kz = 0 and N/2 bins
 // dropped as a C2R transform does), the window minimum, one atomicMin per
 // workgroup.  The product spectra make one HBM round trip, of the window's
-// y rows only.
+// y rows only.  Bound by latency: how many wavefronts the tile's LDS and the
+// registers let run.  So the transforms trade values between lanes
+// (lane_fft), with no LDS and no barrier, and the tile holds x' in two turns.
+// Alone per search, with the whole tile overlaying the transforms' LDS
+// scratch (two of three wavefronts transforming at a time at 96) before: 96
+// (2,000 poses) 2.34 -> 2.31 ms, 128 (1,000) 2.41 -> 2.03; the small tile
+// also fits beside the forward kernel's workgroups: the overlapped searches
+// 9.2 -> 8.8 and 10.8 -> 10.45 ms.  The whole tile with lane_fft: 2.00 / 2.44
+// alone, 9.2 / 11.1 overlapped.
 template <>
 __device__ __forceinline__ unsigned atom_tw_bytes<96>(unsigned k, unsigned i) {
   const unsigned t = mul_u24(k, i);
@@ -2674,9 +2682,9 @@ template <int N>
 struct AtomRows {
   using RS = RegShape<N>;
   static constexpr int ENT = 512;           // staged channel-list entries
-  // Row stride of the LDS tiles (float2), odd: consecutive lines (the
-  // Stockham passes' consecutive threads, and the x-z kernel's lines ln of
-  // one 8-byte access) fall on distinct bank pairs.
+  // Row strides of the LDS tiles (float2; TS and XTS), odd: consecutive lines
+  // (the Stockham passes' consecutive threads, and the x-z kernel's lines ln
+  // of one 8-byte access) fall on distinct bank pairs.
   static constexpr int TS = N + 1;
   static constexpr int STAGE = ENT * 4 + 2 * 4 * 64 * 2;  // ef, ei and the shared operands (float2)
   static constexpr int TILES = 2 * 16 * TS;               // two tiles of 16 lines (Stockham ping-pong)
@@ -2684,12 +2692,13 @@ struct AtomRows {
   static_assert(U % 2 == 0, "float4 storage");
   // k_atoms_xz
   static constexpr int XW = N / 2 / RS::LPW;     // wavefronts
-  static constexpr int XRW = N == 96 ? 2 : XW;   // of them transforming at a time
-  static constexpr int XT = (N / 2 + 1) * TS;    // [kz][x'] tile
-  static constexpr int XU = XT > XRW * RS::SLICE ? XT : XRW * RS::SLICE;
-  // wavefronts per SIMD the tile's LDS allows (160 KB per CU): the compiler
-  // may spend registers up to that occupancy on loads in flight
-  static constexpr int XOCC = (160 * 1024 / (XU * 8 + 2048)) * XW / 4;
+  static constexpr int XHW = (XW + 1) / 2;       // of them reading z lines in the first turn
+  static constexpr int XHX = 2 * RS::LPW * XHW;  // their x' columns
+  static constexpr int XTS = XHX + 1;
+  static constexpr int XU = (N / 2 + 1) * XTS;   // [kz][x'] tile
+  // wavefronts per SIMD to hold the registers to (128 and 80 of them): the
+  // tile (25 and 34 KB) lets about as many run
+  static constexpr int XOCC = N == 96 ? 4 : 6;
 };
 
 template <class P, int PR>
@@ -2789,7 +2798,7 @@ __global__ __launch_bounds__(256) void k_atoms_fwd(const PoseSlot* __restrict__ 
 }
 
 template <class P>
-__global__ __launch_bounds__(64 * AtomRows<P::N>::XW) __attribute__((amdgpu_waves_per_eu(1, AtomRows<P::N>::XOCC)))
+__global__ __launch_bounds__(64 * AtomRows<P::N>::XW) __attribute__((amdgpu_waves_per_eu(AtomRows<P::N>::XOCC, AtomRows<P::N>::XOCC)))
 void k_atoms_xz(const RotMeta* __restrict__ meta,
                                                                       const float2* __restrict__ R,
                                                                       unsigned long long* __restrict__ keys,
@@ -2799,8 +2808,8 @@ void k_atoms_xz(const RotMeta* __restrict__ meta,
   using AR = AtomRows<N>;
   using RS = RegShape<N>;
   constexpr int L = RS::L, V = RS::V, LPW = RS::LPW;
-  constexpr int TS = AR::TS, XRW = AR::XRW, TURNS = (AR::XW + AR::XRW - 1) / AR::XRW;
-  extern __shared__ float2 tb[];  // [ZH][TS] (kz, x'), or the transforms' scratch
+  constexpr int HW = AR::XHW, HX = AR::XHX, TS = AR::XTS;
+  extern __shared__ float2 tb[];  // [ZH][TS] (kz, x')
   __shared__ float2 stwr[L * V];
   const int y = blockIdx.x, s = blockIdx.y;
   const RotMeta m = meta[s];
@@ -2834,48 +2843,52 @@ void k_atoms_xz(const RotMeta* __restrict__ meta,
     }
   }
   __syncthreads();  // stwr
-#pragma unroll
-  for (int r = 0; r < TURNS; ++r) {
-    if (wave / XRW == r) reg_fft<N, 1>(v, twr, tb + (wave % XRW) * RS::SLICE, ln, n2);
-    __syncthreads();  // this turn's scratch reads are done (the [kz][x'] tile overlays the scratch)
-  }
-  // every x' into [kz][x'] (the columns past the window are read as the
-  // partners of the window's last pair); line 0 holds kz = 0 in its real
-  // and kz = N/2 in its imaginary parts
-#pragma unroll
-  for (int j = 0; j < V; ++j) tb[t * TS + n2 + L * j] = v[j];
-  if (t == 0) {
-#pragma unroll
-    for (int j = 0; j < V; ++j) tb[(N / 2) * TS + n2 + L * j] = make_float2(v[j].y, 0.f);
-  }
-  __syncthreads();
+  lane_fft<N, 1>(v, twr);
   // z lines: x' pair (2p, 2p + 1), p = t, as one complex line A + iB; value j
-  // at kz = n2 + L j over the full range (kz > N/2 from the conjugates).  A
-  // wavefront whose pairs all lie past the window skips its transforms.
+  // at kz = n2 + L j over the full range (kz > N/2 from the conjugates).  The
+  // x' columns go through [kz][x'] in two turns, HX at a time, those of the
+  // first HW wavefronts' pairs first (the columns past the window are read as
+  // the partners of its last pair); line 0 holds kz = 0 in its real and kz =
+  // N/2 in its imaginary parts.  A wavefront whose pairs all lie past the
+  // window skips its transforms.
   const int p = t;
   const bool act = 2 * p < wx, bact = 2 * p + 1 < wx;
   const bool wact = 2 * LPW * wave < wx;
   float2 z[V];
+  const float2* zl = tb + 2 * p - (wave >= HW ? HX : 0);
+  auto read = [&] {
 #pragma unroll
-  for (int j = 0; j < V; ++j) {
-    const int k = n2 + L * j;
-    const int kk = k <= N / 2 ? k : N - k;
-    float2 A = tb[kk * TS + 2 * p], B = tb[kk * TS + 2 * p + 1];
-    if (k == 0 || k == N / 2) {
-      A.y = 0.f;
-      B.y = 0.f;
-    } else if (k > N / 2) {
-      A.y = -A.y;
-      B.y = -B.y;
+    for (int j = 0; j < V; ++j) {
+      const int k = n2 + L * j;
+      const int kk = k <= N / 2 ? k : N - k;
+      float2 A = zl[kk * TS], B = zl[kk * TS + 1];
+      if (k == 0 || k == N / 2) {
+        A.y = 0.f;
+        B.y = 0.f;
+      } else if (k > N / 2) {
+        A.y = -A.y;
+        B.y = -B.y;
+      }
+      z[j] = make_float2(A.x - B.y, A.y + B.x);
     }
-    z[j] = make_float2(A.x - B.y, A.y + B.x);
-  }
-  __syncthreads();  // the tile is free: the transforms' scratch
+  };
+  auto put = [&](int h) {
 #pragma unroll
-  for (int r = 0; r < TURNS; ++r) {
-    if (wact && wave / XRW == r) reg_fft<N, 1>(z, twr, tb + (wave % XRW) * RS::SLICE, ln, n2);
-    if (r + 1 < TURNS) __syncthreads();
+    for (int j = 0; j < V; ++j) {
+      if (j / (HX / L) != h) continue;
+      tb[t * TS + n2 + L * j - h * HX] = v[j];
+      if (t == 0) tb[(N / 2) * TS + n2 + L * j - h * HX] = make_float2(v[j].y, 0.f);
+    }
+    __syncthreads();
+  };
+  put(0);
+  if (wx > HX) {  // some pairs of the second turn lie in the window
+    if (wave < HW) read();
+    __syncthreads();  // the first turn's reads are done
+    put(1);
   }
+  if (wx <= HX || wave >= HW) read();
+  if (wact) lane_fft<N, 1>(z, twr);
   // the lane's window minimum: values in increasing translation index (line
   // 2p's z values, then line 2p + 1's); the first strict minimum of the
   // ordered energy bits (the keys' high word) and its position, then one key
@@ -3260,7 +3273,7 @@ hipError_t launch_inv_z(hipStream_t st, int N, const RotMeta* meta, int nslots, 
 }
 
 bool atoms_supported(int N) {
-  // the x-z kernel's tile or scratch (dynamic) and its twiddles and key
+  // the x-z kernel's tile (dynamic) and its twiddles and key
   // reduction (static)
   return N == 64 || ((N == 96 || N == 128) && atoms_xz_lds_bytes(N) + atoms_xz_static_lds(N) <= g_max_dyn_lds);
 }

@@ -551,3 +551,28 @@ def test_atom_form_64_table_edges(ctx, p64, natom):
     assert np.array_equal(mc.view(np.uint32), mb.view(np.uint32))
     prob = orc.PoseProblem(g["values"], g["radii"], g["spacing"], q, e, r)
     check_search(prob, x[None], quats[:2], E[:, :2], idx[:, :2], mc[:, :2])
+
+
+@pytest.mark.parametrize("name,n", [("p96", 96), ("p128", 128)])
+def test_atom_form_96_128_window_edges(ctx, name, n):
+    """96^3 and 128^3 atom form with window widths around the 64 x' columns its
+    x-z kernel takes per turn, and narrow windows: two atoms along x, against
+    the FP64 oracle."""
+    g = workloads.protein_grids(name)
+    prot = cdk.Protein(ctx, g["values"], g["radii"], g["spacing"], g["mid"], g["length"])
+    _, q, e, r = cdk.synth_ligand(811, 2)
+    lig = cdk.Ligand(prot, q, e, r)
+    prob = orc.PoseProblem(g["values"], g["radii"], g["spacing"], q, e, r)
+    quats = np.array([[1, 0, 0, 0]], np.float32)
+    ctx.set_option("pipeline", 2)
+    try:
+        for w in (62, 63, 64, 65, 66, 67, 68, 33, 9):
+            d = (n - w) * g["spacing"]
+            x = np.array([[[0, 0, 0], [d, 0.4, 0.7]]], np.float32)
+            E, idx, mc = cdk.search(ctx, prot, lig, x, quats)
+            say("window edge", name, w, idx[0, 0])
+            check_search(prob, x, quats, E, idx, mc)
+    finally:
+        ctx.set_option("pipeline", -1)
+    lig.close()
+    prot.close()
