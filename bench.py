@@ -841,7 +841,7 @@ def main():
                     help="CPU baseline threads (0 = every usable host core, at most the box's share of 16)")
     ap.add_argument("--no-graph", action="store_true")
     ap.add_argument("--chunk", type=int, default=0, help="poses per fused launch set (0 = from the HBM budget)")
-    ap.add_argument("--group", type=int, default=0, help="poses per mid-kernel workgroup (0 = autotuned)")
+    ap.add_argument("--group", type=int, default=0, help="poses per mid-kernel workgroup (0 = by the launch size)")
     ap.add_argument("--pipeline", type=int, default=-1,
                     help="fused engine form: 0 planes, 1 columns (64^3), 2 atoms (64^3, 96^3, 128^3), -1 autotuned")
     ap.add_argument("--overlap-z", type=int, default=1,

@@ -666,10 +666,11 @@ struct Tuned {
 //    forward and inverse plane stage forms, once per grid size: the forms
 //    round differently, so fixing them per (context, N) keeps results
 //    independent of how poses are batched;
-//  - the mid-stage schedule per launch shape (N, channels, box bound, chunk):
-//    plane form group, ring depth and poses per protein load, column form
-//    group.  Schedules only reorder work; results are bit-identical.
+//  - the column form's group, per (N, channels).
 // Choices are made by timing every candidate twice and keeping the faster.
+// The plane and atom forms' mid-stage schedules follow the launch size
+// (mid_plan, atom_group).  Schedules only reorder work; results are
+// bit-identical.
 Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
   const int N = prot.N;
   Tuned tu;
@@ -677,19 +678,11 @@ Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
   const bool reg_ok = inv_reg_supported(N);
   const bool col_ok = col_supported(N) && prot.spec_kz.p != nullptr;
   const bool atoms_ok = atoms_supported(N) && prot.spec_mf.p != nullptr;
-  // The plane form's schedule is kept per (N, channels, box bound, launch
-  // size rounded up to a power of two): a server's launch sets vary in size
-  // from set to set, and a key per exact size would re-run the tuner on
-  // nearly every set.
-  size_t chunk_class = 1;
-  while (chunk_class < chunk) chunk_class <<= 1;
-  const std::array<int, 4> gkey = {N, t.cmax, t.boxmax, (int)std::min<size_t>(chunk_class, 1 << 30)};
-  // The column and atom forms' group choice is kept per (N, channels): their
-  // best group hardly moves with the box bound or the launch size, and a
-  // server sees a new (box bound, chunk) pair on many launch sets.
+  const int set = (int)std::min(chunk, t.slots.size());  // poses of a full launch set
+  // Kept per (N, channels), not per box bound and launch size: a server sees
+  // a new pair of those on many launch sets.
   const std::array<int, 4> ckey = {N, t.cmax, 0, 0};
-  bool need_pipe = false, need_fwd = false, need_inv = false, need_group = false, need_col = false,
-       need_atom = false;
+  bool need_pipe = false, need_fwd = false, need_inv = false, need_col = false;
   if (ctx.pipeline >= 0) {
     tu.pipe = (ctx.pipeline == kPipeColumns && col_ok)  ? kPipeColumns
               : (ctx.pipeline == kPipeAtoms && atoms_ok) ? kPipeAtoms
@@ -737,16 +730,10 @@ Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
     tu.col_group = ctx.mid_group;
     tu.atom_group = ctx.mid_group;
   } else {
-    if (planes) {
-      auto it = ctx.tuned_group.find(gkey);
-      if (it != ctx.tuned_group.end()) {
-        tu.group = it->second[0];
-        tu.depth = it->second[1];
-        tu.poses = it->second[2];
-      } else {
-        need_group = true;
-      }
-    }
+    const MidPlan mp = mid_plan(N, set);
+    tu.group = mp.group;
+    tu.depth = mp.depth;
+    tu.poses = mp.poses;
     if (cols) {
       auto it = ctx.tuned_col_group.find(ckey);
       if (it != ctx.tuned_col_group.end())
@@ -754,15 +741,9 @@ Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
       else
         need_col = true;
     }
-    if (atoms) {
-      auto it = ctx.tuned_atom_group.find(ckey);
-      if (it != ctx.tuned_atom_group.end())
-        tu.atom_group = it->second;
-      else
-        need_atom = true;
-    }
+    tu.atom_group = atom_group(N, ctx.atom_products, t.astride, set);
   }
-  if (!need_pipe && !need_fwd && !need_inv && !need_group && !need_col && !need_atom) return tu;
+  if (!need_pipe && !need_fwd && !need_inv && !need_col) return tu;
 
   const int n = (int)std::min(chunk, t.slots.size());
   const float2* tw = ctx.twiddle(N);
@@ -823,7 +804,7 @@ Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
   };
   float plane_ms = 0.f, col_ms = 0.f, atom_ms = 0.f;
   try {
-    if (need_fwd || need_inv || need_group || (need_pipe && planes)) {
+    if (need_fwd || need_inv || (need_pipe && planes)) {
       if (need_fwd) {
         const float tb = timed([&] { fwd(kFwdBlock); });
         const float twv = timed([&] { fwd(kFwdReg); });
@@ -833,43 +814,7 @@ Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
       } else {
         plane_ms += timed([&] { fwd(tu.fwd); });
       }
-      if (need_group) {
-        // One pose at a time: group size at the shallowest ring, then the
-        // ring depth at that group.  Then runs of 2 and 4 poses per protein
-        // load over the group sizes.
-        const int d0 = std::min(2, max_depth);
-        float best = 1e30f;
-        for (int g : {4, 8, 16, 32}) {
-          const float ms = mid(g, d0, 1);
-          if (ms < best) {
-            best = ms;
-            tu.group = g;
-          }
-        }
-        tu.depth = d0;
-        for (int d = d0 + 1; d <= max_depth; ++d) {
-          const float ms = mid(tu.group, d, 1);
-          if (ms < best) {
-            best = ms;
-            tu.depth = d;
-          }
-        }
-        tu.poses = 1;
-        for (int np = 2; np <= max_poses; np *= 2)
-          for (int g : {4, 8, 16, 32}) {
-            const float ms = mid(g, tu.depth, np);
-            if (ms < best) {
-              best = ms;
-              tu.group = g;
-              tu.poses = np;
-            }
-          }
-        if (ctx.tuned_group.size() >= kMaxTunedShapes) ctx.tuned_group.erase(ctx.tuned_group.begin());
-        ctx.tuned_group[gkey] = {tu.group, tu.depth, tu.poses};
-        plane_ms += best;
-      } else {
-        plane_ms += mid(tu.group, tu.depth, tu.poses);
-      }
+      plane_ms += mid(tu.group, tu.depth, tu.poses);
       if (need_inv) {
         const float tb = timed([&] { inv(kInvBlock); });
         const float tr = timed([&] { inv(kInvReg); });
@@ -904,21 +849,13 @@ Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
         hip_check(launch_inv_z(ctx.stream, N, d_meta, n, ctx.w_T, d_keys, tw), "tune column inverse");
       });
     }
-    if (need_atom || (need_pipe && atoms)) {
-      auto mida = [&](int g) {
-        return timed([&] {
-          hip_check(launch_mid_atoms(ctx.stream, N, sl, d_ligs, t.d_pad.as<int>(), t.d_wv.as<float>(),
-                                     t.d_wq.as<float>(), ctx.w_ag, t.astride, d_meta, n, g,
-                                     prot.spec_mf.as<float2>(), ctx.w_T, invG, tw, ctx.atom_products),
-                    "tune atom mid");
-        });
-      };
-      if (need_atom) {
-        atom_ms += best_group(mida, tu.atom_group);
-        ctx.tuned_atom_group[ckey] = tu.atom_group;
-      } else {
-        atom_ms += mida(tu.atom_group);
-      }
+    if (need_pipe && atoms) {
+      atom_ms += timed([&] {
+        hip_check(launch_mid_atoms(ctx.stream, N, sl, d_ligs, t.d_pad.as<int>(), t.d_wv.as<float>(),
+                                   t.d_wq.as<float>(), ctx.w_ag, t.astride, d_meta, n, tu.atom_group,
+                                   prot.spec_mf.as<float2>(), ctx.w_T, invG, tw, ctx.atom_products),
+                  "tune atom mid");
+      });
       atom_ms += timed([&] {
         hip_check(launch_inv_z(ctx.stream, N, d_meta, n, ctx.w_T, d_keys, tw), "tune atom inverse");
       });
@@ -976,7 +913,6 @@ void enqueue_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk,
   unsigned long long* d_keys = t.d_keys.as<unsigned long long>();
   RotMeta* d_meta = t.d_meta.as<RotMeta>();
   const size_t total = t.slots.size();
-  const int group = std::max(1, tu.group);
   const bool ovl = overlap_z_stage(ctx, tu);
   size_t last_set = 0;
   for (size_t s = 0; s < total; s += chunk) {
@@ -996,7 +932,8 @@ void enqueue_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk,
       if (ovl && si >= 2) hip_check(hipStreamWaitEvent(ctx.stream, ctx.set_events[2 * (si - 2) + 1], 0), "wait");
       e = timer.begin(2);
       hip_check(launch_mid_atoms(ctx.stream, N, sl, d_ligs, t.d_pad.as<int>(), t.d_wv.as<float>(),
-                                 t.d_wq.as<float>(), ctx.w_ag, t.astride, d_meta + s, n, tu.atom_group,
+                                 t.d_wq.as<float>(), ctx.w_ag, t.astride, d_meta + s, n,
+                                 ctx.mid_group > 0 ? ctx.mid_group : atom_group(N, ctx.atom_products, t.astride, n),
                                  prot.spec_mf.as<float2>(), T2, 1.0f / (float)G, tw, ctx.atom_products),
                 "atom mid");
       timer.end(e);
@@ -1038,7 +975,8 @@ void enqueue_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk,
               "fwd planes");
     timer.end(e);
     e = timer.begin(2);
-    hip_check(launch_mid(ctx.stream, N, tu.depth, tu.poses, sl, d_ligs, d_meta + s, n, group, ctx.w_A, t.cmax,
+    const MidPlan mp = ctx.mid_group > 0 ? MidPlan{tu.group, tu.depth, tu.poses} : mid_plan(N, n);
+    hip_check(launch_mid(ctx.stream, N, mp.depth, mp.poses, sl, d_ligs, d_meta + s, n, mp.group, ctx.w_A, t.cmax,
                          t.boxmax,
                          prot.spec_lb.as<float2>(), prot.nch, ctx.w_T, 1.0f / (float)G, tw),
               "mid");

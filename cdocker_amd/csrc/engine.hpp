@@ -241,17 +241,12 @@ struct Context {
   // Autotuner state.  The forward and inverse plane forms change FFT
   // rounding, so each is chosen once per grid size and kept for the
   // context's life (results then do not depend on how poses are batched);
-  // the mid group size only changes the schedule and is tuned per launch
-  // shape, with the ring depth and the poses per protein load.
+  // the mid group size only changes the schedule.
   size_t max_dyn_lds = 64 * 1024;
   std::map<int, int> tuned_pipe;                     // N -> pipeline form
   std::map<int, int> tuned_fwd;                      // N -> variant
   std::map<int, int> tuned_inv;                      // N -> variant
-  // (N, cmax, boxmax, chunk rounded up to a power of two) -> (group, depth,
-  // poses per protein load)
-  std::map<std::array<int, 4>, std::array<int, 3>> tuned_group;
   std::map<std::array<int, 4>, int> tuned_col_group;   // (N, cmax, 0, 0) -> column form group
-  std::map<std::array<int, 4>, int> tuned_atom_group;  // (N, cmax, 0, 0) -> atom form group
   int last_fwd = -1, last_inv = -1, last_group = 0, last_depth = 0, last_poses = 0,
       last_pipe = -1;
   StageTimes stage_times;

@@ -3278,6 +3278,26 @@ bool atoms_supported(int N) {
   return N == 64 || ((N == 96 || N == 128) && atoms_xz_lds_bytes(N) + atoms_xz_static_lds(N) <= g_max_dyn_lds);
 }
 
+// Poses per workgroup of the atom form's mid stage.  A workgroup that runs
+// several in turn saves its set-up (twiddles, tables' addresses) once the
+// launch is many times what runs at a time; a shorter launch is over sooner
+// with one pose per workgroup.  x = workgroups of one pose each / resident
+// ones.  Measured, us of 1 / 2 / 4 poses per workgroup: 64 (24 atoms) 10 poses
+// (x = 0.3) 24 / 38 / 70, 50 (1.7) 63 / 60 / 76, 200 (6.6) 190 / 191 / 203,
+// 500 (17) 461 / 441 / 447; 64 (100 atoms) 20 (0.6) 56 / 74 / 105, 400 (13)
+// 783 / 752 / 739; 96 8 (0.9) 45 / 60 / 91, 64 (7.4) 257 / 258 / 263, 128 (15)
+// 533 / 496 / 482; 128 8 (2.0) 93 / 107 / 125, 32 (8.1) 334 / 332 / 331, 64
+// (16) 677 / 618 / 595.  8 is nowhere faster than 4 by more than 2%.
+int atom_group(int N, int products, int astride, int nslots) {
+  const int ZH = N / 2 + 1;
+  const bool x3 = N == 64 && products == kAtomF16x3 && astride <= AtomTab::ROWS;
+  // workgroups per pose, and resident per CU (256 of them)
+  const int items = x3 ? (ZH + AtomTab::NP - 1) / AtomTab::NP : N == 64 ? ZH : ZH * (N / 32);
+  const int per_cu = x3 ? 2 : N == 96 ? 5 : 4;
+  const double x = (double)items * nslots / (256 * per_cu);
+  return x >= 12 ? 4 : x >= 6 ? 2 : 1;
+}
+
 hipError_t launch_mid_atoms(hipStream_t st, int N, const PoseSlot* slots, const LigandDesc* ligs,
                             const int* pad_atoms, const float* wv, const float* wq, const AtomGrid* ag, int astride,
                             const RotMeta* meta, int nslots, int group, const float2* P3, float2* T2, float invG,
@@ -3396,6 +3416,24 @@ void mid_np_launch_one(dim3 grid, hipStream_t st, const PoseSlot* slots, const L
 
 int mid_max_depth(int N) { return (N == 32 || N == 64) ? 3 : 1; }
 int mid_max_poses(int N) { return (N == 32 || N == 64) ? 4 : 1; }
+
+// One pose per workgroup and no sharing is the fastest nearly everywhere: the
+// protein spectra come from the XCD's L2 and a workgroup has little to set up,
+// so longer runs only lengthen the launch's tail.  Measured, us of 1 / 4 / 32
+// poses per workgroup: 48 (24 atoms) 20 poses 17 / 42 / 187, 500 283 / 300 /
+// 462, 4,000 1,023 / 1,031 / 1,116 per launch; 32 (16 atoms) 20 poses 11 / 27 /
+// 110, 2,000 332 / 338 / 444; 96 (40 atoms) of 1 / 2 / 4: 20 poses 83 / 88 /
+// 99, 200 818 / 809 / 814.  The two exceptions: at 64 two poses per protein
+// load, run two at a time, once the launch fills the chip (5 poses 15 against
+// 18, 20 26.5 / 25.4, 100 155 / 133, 500 685 / 569); and at 128 four poses per
+// workgroup in long launches (20 poses 238 against 273, 60 786 / 726).  The
+// ring's third buffer and four poses per load win nowhere.
+MidPlan mid_plan(int N, int nslots) {
+  const int depth = mid_max_depth(N) < 2 ? mid_max_depth(N) : 2;
+  if (N == 64 && nslots >= 16) return {2, depth, 2};
+  if (N == 128 && nslots >= 40) return {4, depth, 1};
+  return {1, depth, 1};
+}
 
 hipError_t launch_mid(hipStream_t st, int N, int depth, int np, const PoseSlot* slots, const LigandDesc* ligs,
                       const RotMeta* meta, int nslots, int group, const float2* A, int cmax, int boxmax,

@@ -52,6 +52,11 @@ hipError_t launch_fwd_planes(hipStream_t st, int N, int variant, const PoseSlot*
 // (depth, np, group) gives bit-identical results.
 int mid_max_depth(int N);
 int mid_max_poses(int N);
+// The schedule launch_mid should get for a launch of nslots poses.
+struct MidPlan {
+  int group, depth, poses;
+};
+MidPlan mid_plan(int N, int nslots);
 hipError_t launch_mid(hipStream_t st, int N, int depth, int np, const PoseSlot* slots, const LigandDesc* ligs,
                       const RotMeta* meta, int nslots, int group, const float2* A, int cmax, int boxmax,
                       const float2* Phat, int npch, float2* T, float invG, const float2* tw);
@@ -93,6 +98,9 @@ bool atoms_supported(int N);
 constexpr int kAtomF16 = 0, kAtomF32 = 1, kAtomF16x3 = 2;
 constexpr float kAtomYScale = 4096.f;
 // pad_atoms: the ligands' padded channel lists (LigandDesc::pad_atoms).
+// The group launch_mid_atoms should get for a launch of nslots poses of
+// ligands of at most astride atoms.
+int atom_group(int N, int products, int astride, int nslots);
 hipError_t launch_mid_atoms(hipStream_t st, int N, const PoseSlot* slots, const LigandDesc* ligs,
                             const int* pad_atoms, const float* wv, const float* wq, const AtomGrid* ag, int astride,
                             const RotMeta* meta, int nslots, int group, const float2* P3, float2* T2, float invG,

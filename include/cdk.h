@@ -55,7 +55,7 @@ int cdk_context_create(int device, cdk_context** out);
 int cdk_context_destroy(cdk_context* ctx);
 /* Options: "ws_budget_bytes", "ref_batch" (B, default 50 as NoMini:208),
  * "fused_chunk" (poses per fused launch set, 0 = from budget), "mid_group"
- * (poses per mid-stage workgroup, 0 = autotuned with the ring depth),
+ * (poses per mid-stage workgroup, 0 = by the size of the launch),
  * "mid_depth" (register buffers in the mid stage's (pose, channel) ring when
  * mid_group is fixed: 2 or 3 at 32^3/64^3, 0 = 2), "mid_poses" (poses of
  * one ligand that share each protein spectrum load when mid_group is fixed:
@@ -83,7 +83,7 @@ int cdk_context_destroy(cdk_context* ctx);
 int cdk_context_set_option(cdk_context* ctx, const char* key, int64_t value);
 /* Reads an option back; also "last_fwd_variant", "last_inv_variant",
  * "last_pipeline", "last_mid_group", "last_mid_depth" and "last_mid_poses"
- * (what the autotuner chose for the last fused search), "max_dyn_lds" (the
+ * (what the last fused search ran with), "max_dyn_lds" (the
  * device's dynamic LDS limit per workgroup, bytes) and "workspace_bytes"
  * (device bytes of the fused engine's launch-set working arrays: one pool,
  * carved per search; never above "ws_budget_bytes" unless "fused_chunk"

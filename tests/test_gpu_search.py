@@ -576,3 +576,29 @@ def test_atom_form_96_128_window_edges(ctx, name, n):
         ctx.set_option("pipeline", -1)
     lig.close()
     prot.close()
+
+
+@pytest.mark.parametrize("pipe,sizes", [(2, {1: 1, 180: 1, 181: 2, 361: 2, 362: 4}), (0, {1: 1, 15: 1, 16: 2, 17: 2})])
+def test_schedule_follows_launch_size(ctx, p64, pipe, sizes):
+    """64^3 atom and plane forms on both sides of each launch size where the
+    mid stage's schedule changes, after a large search: the schedule is the
+    size's own, and the results are bit-identical to a fixed one's."""
+    g, prot = p64
+    x, q, e, r = cdk.synth_ligand(821, 9)
+    lig = cdk.Ligand(prot, q, e, r)
+    quats = cdk.QuaternionUniformSampling(cdk.Rng(23), 2000)
+    ctx.set_option("pipeline", pipe)
+    try:
+        cdk.search(ctx, prot, lig, x[None], quats)
+        for n, group in sizes.items():
+            say("schedule pipe=%d n=%d" % (pipe, n))
+            E, idx, mc = cdk.search(ctx, prot, lig, x[None], quats[:n])
+            assert ctx.get_option("last_mid_group") == group
+            ctx.set_option("mid_group", 3)
+            Ef, ixf, mcf = cdk.search(ctx, prot, lig, x[None], quats[:n])
+            ctx.set_option("mid_group", 0)
+            assert np.array_equal(E.view(np.uint32), Ef.view(np.uint32)) and np.array_equal(idx, ixf)
+            assert np.array_equal(mc.view(np.uint32), mcf.view(np.uint32))
+    finally:
+        ctx.set_option("mid_group", 0)
+        ctx.set_option("pipeline", -1)
