@@ -3417,20 +3417,23 @@ void mid_np_launch_one(dim3 grid, hipStream_t st, const PoseSlot* slots, const L
 int mid_max_depth(int N) { return (N == 32 || N == 64) ? 3 : 1; }
 int mid_max_poses(int N) { return (N == 32 || N == 64) ? 4 : 1; }
 
-// One pose per workgroup and no sharing is the fastest nearly everywhere: the
+// One pose per workgroup and no sharing is the fastest in short launches: the
 // protein spectra come from the XCD's L2 and a workgroup has little to set up,
 // so longer runs only lengthen the launch's tail.  Measured, us of 1 / 4 / 32
 // poses per workgroup: 48 (24 atoms) 20 poses 17 / 42 / 187, 500 283 / 300 /
-// 462, 4,000 1,023 / 1,031 / 1,116 per launch; 32 (16 atoms) 20 poses 11 / 27 /
-// 110, 2,000 332 / 338 / 444; 96 (40 atoms) of 1 / 2 / 4: 20 poses 83 / 88 /
-// 99, 200 818 / 809 / 814.  The two exceptions: at 64 two poses per protein
-// load, run two at a time, once the launch fills the chip (5 poses 15 against
-// 18, 20 26.5 / 25.4, 100 155 / 133, 500 685 / 569); and at 128 four poses per
-// workgroup in long launches (20 poses 238 against 273, 60 786 / 726).  The
-// ring's third buffer and four poses per load win nowhere.
+// 462, 4,000 1,023 / 1,031 / 1,116 per launch; 96 (40 atoms) of 1 / 2 / 4: 20
+// poses 83 / 88 / 99, 200 818 / 809 / 814.  Two poses per protein load, run two
+// at a time, win at 32 and 64 once the launch fills the chip: 64 (24 atoms) 5
+// poses 15 against 18, 20 26.5 / 25.4, 100 155 / 133, 500 685 / 569; 32 of one
+// pose / two shared (16 atoms) 300 poses 39 / 41, 500 58 / 58, 1,000 146 / 127,
+// 4,000 574 / 475, 150,000 20.3 / 17.0 ms; (30 atoms) 300 39 / 42, 500 73 / 66,
+// 12,000 1,774 / 1,469; (8 atoms) 500 49 / 49, 1,000 94 / 89, 12,000 1,367 /
+// 1,132.  At 128 four poses per workgroup win in long launches (20 poses 238
+// against 273, 60 786 / 726).  The ring's third buffer and four poses per load
+// win nowhere.
 MidPlan mid_plan(int N, int nslots) {
   const int depth = mid_max_depth(N) < 2 ? mid_max_depth(N) : 2;
-  if (N == 64 && nslots >= 16) return {2, depth, 2};
+  if ((N == 64 && nslots >= 16) || (N == 32 && nslots >= 500)) return {2, depth, 2};
   if (N == 128 && nslots >= 40) return {4, depth, 1};
   return {1, depth, 1};
 }

@@ -602,3 +602,30 @@ def test_schedule_follows_launch_size(ctx, p64, pipe, sizes):
     finally:
         ctx.set_option("mid_group", 0)
         ctx.set_option("pipeline", -1)
+
+
+@pytest.mark.parametrize("n,poses", [(1, 1), (499, 1), (500, 2), (501, 2)])
+def test_schedule_32_shares_protein_loads(ctx, n, poses):
+    """32^3 on both sides of the launch size from which two poses share each
+    protein load, an odd count among them: the sharing is on, and the results
+    are bit-identical to one pose at a time."""
+    vals, radii, mid, ln = cdk.synth_protein(15, 900, 16.0, 32, 0.5)
+    prot = cdk.Protein(ctx, vals, radii, 0.5, mid, ln)
+    x, q, e, r = cdk.synth_ligand(831, 8)
+    x = (x * np.float32(0.5)).astype(np.float32)
+    lig = cdk.Ligand(prot, q, e, r)
+    quats = cdk.QuaternionUniformSampling(cdk.Rng(29), 501)[:n]
+    say("schedule 32^3 n=%d" % n)
+    try:
+        E, idx, mc = cdk.search(ctx, prot, lig, x[None], quats)
+        assert ctx.get_option("last_mid_poses") == poses
+        ctx.set_option("mid_group", 1)
+        Ef, ixf, mcf = cdk.search(ctx, prot, lig, x[None], quats)
+        assert ctx.get_option("last_mid_poses") == 1
+    finally:
+        ctx.set_option("mid_group", 0)
+        lig.close()
+        prot.close()
+    assert np.isfinite(E).any()
+    assert np.array_equal(E.view(np.uint32), Ef.view(np.uint32)) and np.array_equal(idx, ixf)
+    assert np.array_equal(mc.view(np.uint32), mcf.view(np.uint32))
