@@ -655,97 +655,82 @@ void ensure_fused_work(Context& ctx, const Protein& prot, const Prepared& t, siz
 
 struct Tuned {
   int pipe = kPipePlanes;
-  int fwd = kFwdBlock, inv = kInvBlock, group = 16, depth = 1, poses = 1;  // plane form
-  int col_group = 4;                                                       // column form
-  int atom_group = 4;                                                      // atom form
+  int fwd = kFwdBlock, inv = kInvBlock, group = 1, depth = 1, poses = 1;  // plane form
+  int col_group = 1;                                                      // column form
+  int atom_group = 1;                                                     // atom form
   int mid_group() const { return pipe == kPipeColumns ? col_group : pipe == kPipeAtoms ? atom_group : group; }
 };
 
-// Autotuner, on the first launch set of a search:
-//  - the pipeline form (plane or column form) and, for the plane form, the
-//    forward and inverse plane stage forms, once per grid size: the forms
-//    round differently, so fixing them per (context, N) keeps results
-//    independent of how poses are batched;
-//  - the column form's group, per (N, channels).
-// Choices are made by timing every candidate twice and keeping the faster.
-// The plane and atom forms' mid-stage schedules follow the launch size
-// (mid_plan, atom_group).  Schedules only reorder work; results are
-// bit-identical.
+// Searches whose largest ligand has at most this many atoms take the atom form
+// where it is supported, untimed (with FP16 products): it is the fastest for
+// them at every edge and launch size.  Measured, us of a call, atom / best other form: 64 24 atoms, 1
+// pose 74 / 80, 1,000 1,040 / 1,573; 84 atoms, 20 105 / 252, 400 531 / 1,075;
+// 96 40 atoms, 1 93 / 179, 1,000 5,150 / 9,979; 84 atoms, 400 2,769 / 7,090;
+// 128 50 atoms, 1 94 / 202, 1,000 10.9 / 29.6 ms; at worst 64 with one atom, 200
+// poses 10% behind the column form.  Above it the line depends on the ligand's
+// extent: 64, 400 poses, 100 atoms in a chain 837 / 1,431, in a ball of 11 A
+// 881 / 743; 200 in a ball 1,410 / 835; 96 4,941 / 4,130.
+constexpr int kAtomFormAtoms = 84;
+
+// The forms and the first launch set's schedule of a search.
+//  - The pipeline form, once per grid size: the forms round differently, so
+//    one per (context, N) keeps results independent of how poses are batched.
+//    Searches of larger ligands than kAtomFormAtoms time the forms on their
+//    first launch set, twice each, and keep the fastest.
+//  - The plane form's forward and inverse stages, which round differently too,
+//    by the grid edge.  Measured, us of block / register transforms: 32 (16
+//    atoms) forward 20 poses 24 / 23, 4,000 326 / 397, inverse 10 / 21 and 311 /
+//    767; 48 (60 atoms) 151 / 157, 3,536 / 5,008 and 10 / 24, 244 / 820; 64 (24
+//    atoms) 77 / 51, 4,000 2,586 / 2,668 and 24 / 20, 2,232 / 1,457; 96 (40)
+//    1,000 2,755 / 2,140 and 3,571 / 2,689; 128 (50) 10.0 / 6.2 ms and 13.4 /
+//    7.3 ms.
+//  - The mid stage's schedule by launch size (mid_plan, atom_group); the column
+//    form runs one pose per workgroup (24 atoms, us of 1 / 2 / 4 / 8: 10 poses
+//    31 / 44 / 84 / 161, 200 207 / 213 / 236 / 274, 8,000 1,578 / 1,584 / 1,571
+//    / 1,606 per launch set).  Schedules only reorder work; results are
+//    bit-identical.
 Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
   const int N = prot.N;
   Tuned tu;
-  const bool fwd_reg_ok = fwd_reg_supported(N);
-  const bool reg_ok = inv_reg_supported(N);
   const bool col_ok = col_supported(N) && prot.spec_kz.p != nullptr;
   const bool atoms_ok = atoms_supported(N) && prot.spec_mf.p != nullptr;
-  const int set = (int)std::min(chunk, t.slots.size());  // poses of a full launch set
-  // Kept per (N, channels), not per box bound and launch size: a server sees
-  // a new pair of those on many launch sets.
-  const std::array<int, 4> ckey = {N, t.cmax, 0, 0};
-  bool need_pipe = false, need_fwd = false, need_inv = false, need_col = false;
+  const int n = (int)std::min(chunk, t.slots.size());  // poses of a full launch set
+  tu.fwd = (ctx.fwd_variant >= 0 ? ctx.fwd_variant == kFwdReg : N >= 64) && fwd_reg_supported(N) ? kFwdReg : kFwdBlock;
+  tu.inv = (ctx.inv_variant >= 0 ? ctx.inv_variant == kInvReg : N >= 64) && inv_reg_supported(N) ? kInvReg : kInvBlock;
+  if (ctx.mid_group > 0) {
+    const int max_depth = mid_max_depth(N);
+    tu.group = ctx.mid_group;
+    tu.depth = ctx.mid_depth > 0 ? std::min(ctx.mid_depth, max_depth) : std::min(2, max_depth);
+    tu.poses = ctx.mid_poses > 0 ? std::min(ctx.mid_poses, mid_max_poses(N)) : 1;
+    tu.col_group = ctx.mid_group;
+    tu.atom_group = ctx.mid_group;
+  } else {
+    const MidPlan mp = mid_plan(N, n);
+    tu.group = mp.group;
+    tu.depth = mp.depth;
+    tu.poses = mp.poses;
+    tu.atom_group = atom_group(N, ctx.atom_products, t.astride, n);
+  }
   if (ctx.pipeline >= 0) {
     tu.pipe = (ctx.pipeline == kPipeColumns && col_ok)  ? kPipeColumns
               : (ctx.pipeline == kPipeAtoms && atoms_ok) ? kPipeAtoms
                                                          : kPipePlanes;
-  } else {
-    auto it = ctx.tuned_pipe.find(N);
-    if (it != ctx.tuned_pipe.end())
-      tu.pipe = it->second;
-    else if (col_ok || atoms_ok)
-      need_pipe = true;
-    else
-      ctx.tuned_pipe[N] = tu.pipe = kPipePlanes;
+    return tu;
   }
-  const bool planes = need_pipe || tu.pipe == kPipePlanes;
-  const bool cols = (need_pipe && col_ok) || tu.pipe == kPipeColumns;
-  const bool atoms = (need_pipe && atoms_ok) || tu.pipe == kPipeAtoms;
-  if (ctx.inv_variant >= 0) {
-    tu.inv = (ctx.inv_variant == kInvReg && reg_ok) ? kInvReg : kInvBlock;
-  } else {
-    auto it = ctx.tuned_inv.find(N);
-    if (it != ctx.tuned_inv.end())
-      tu.inv = it->second;
-    else if (reg_ok)
-      need_inv = planes;
-    else
-      ctx.tuned_inv[N] = tu.inv = kInvBlock;
+  auto it = ctx.tuned_pipe.find(N);
+  if (it != ctx.tuned_pipe.end()) {
+    tu.pipe = it->second;
+    return tu;
   }
-  if (ctx.fwd_variant >= 0) {
-    tu.fwd = (ctx.fwd_variant == kFwdReg && fwd_reg_ok) ? kFwdReg : kFwdBlock;
-  } else {
-    auto it = ctx.tuned_fwd.find(N);
-    if (it != ctx.tuned_fwd.end())
-      tu.fwd = it->second;
-    else if (fwd_reg_ok)
-      need_fwd = planes;
-    else
-      ctx.tuned_fwd[N] = tu.fwd = kFwdBlock;
+  if (!col_ok && !atoms_ok) {
+    ctx.tuned_pipe[N] = tu.pipe = kPipePlanes;
+    return tu;
   }
-  const int max_depth = mid_max_depth(N);
-  const int max_poses = mid_max_poses(N);
-  if (ctx.mid_group > 0) {
-    tu.group = ctx.mid_group;
-    tu.depth = ctx.mid_depth > 0 ? std::min(ctx.mid_depth, max_depth) : std::min(2, max_depth);
-    tu.poses = ctx.mid_poses > 0 ? std::min(ctx.mid_poses, max_poses) : 1;
-    tu.col_group = ctx.mid_group;
-    tu.atom_group = ctx.mid_group;
-  } else {
-    const MidPlan mp = mid_plan(N, set);
-    tu.group = mp.group;
-    tu.depth = mp.depth;
-    tu.poses = mp.poses;
-    if (cols) {
-      auto it = ctx.tuned_col_group.find(ckey);
-      if (it != ctx.tuned_col_group.end())
-        tu.col_group = it->second;
-      else
-        need_col = true;
-    }
-    tu.atom_group = atom_group(N, ctx.atom_products, t.astride, set);
+  if (atoms_ok && ctx.atom_products != kAtomF32 && t.astride <= kAtomFormAtoms) {
+    ctx.tuned_pipe[N] = tu.pipe = kPipeAtoms;
+    return tu;
   }
-  if (!need_pipe && !need_fwd && !need_inv && !need_col) return tu;
 
-  const int n = (int)std::min(chunk, t.slots.size());
   const float2* tw = ctx.twiddle(N);
   const PoseSlot* sl = t.d_slots.as<PoseSlot>();
   const LigandDesc* d_ligs = t.d_ligs.as<LigandDesc>();
@@ -771,108 +756,55 @@ Tuned tune_fused(Context& ctx, const Protein& prot, Prepared& t, size_t chunk) {
     }
     return best;
   };
-  // The fastest of the group sizes 1, 2, 4, 8 for a mid stage: three
-  // round-robin passes, each size's minimum, so clock ramps and the order of
-  // the trials do not pick the size.
-  auto best_group = [&](auto&& time_group, int& group) {
-    const int sizes[4] = {1, 2, 4, 8};
-    float t[4] = {1e30f, 1e30f, 1e30f, 1e30f};
-    for (int pass = 0; pass < 3; ++pass)
-      for (int i = 0; i < 4; ++i) t[i] = std::min(t[i], time_group(sizes[i]));
-    int b = 0;
-    for (int i = 1; i < 4; ++i)
-      if (t[i] < t[b]) b = i;
-    group = sizes[b];
-    return t[b];
-  };
-  auto fwd = [&](int variant) {
-    hip_check(launch_fwd_planes(ctx.stream, N, variant, sl, n, d_ligs, t.d_chan.as<int>(), t.d_wv.as<float>(),
-                                t.d_wq.as<float>(), ctx.w_ag, t.astride, d_meta, t.cmax, t.boxmax,
-                                t.max_chan_atoms, ctx.w_A, tw),
-              "tune fwd planes");
-  };
-  auto mid = [&](int g, int depth, int np) {
-    return timed([&] {
-      hip_check(launch_mid(ctx.stream, N, depth, np, sl, d_ligs, d_meta, n, g, ctx.w_A, t.cmax,
+  try {
+    tu.pipe = kPipePlanes;
+    float best = timed([&] {
+      hip_check(launch_fwd_planes(ctx.stream, N, tu.fwd, sl, n, d_ligs, t.d_chan.as<int>(), t.d_wv.as<float>(),
+                                  t.d_wq.as<float>(), ctx.w_ag, t.astride, d_meta, t.cmax, t.boxmax,
+                                  t.max_chan_atoms, ctx.w_A, tw),
+                "tune fwd planes");
+    });
+    best += timed([&] {
+      hip_check(launch_mid(ctx.stream, N, tu.depth, tu.poses, sl, d_ligs, d_meta, n, tu.group, ctx.w_A, t.cmax,
                            t.boxmax, prot.spec_lb.as<float2>(), prot.nch, ctx.w_T, invG, tw),
                 "tune mid");
     });
-  };
-  auto inv = [&](int variant) {
-    hip_check(launch_inv_argmin(ctx.stream, N, variant, d_meta, n, N - 2, ctx.w_T, d_keys, tw),
-              "tune inverse");
-  };
-  float plane_ms = 0.f, col_ms = 0.f, atom_ms = 0.f;
-  try {
-    if (need_fwd || need_inv || (need_pipe && planes)) {
-      if (need_fwd) {
-        const float tb = timed([&] { fwd(kFwdBlock); });
-        const float twv = timed([&] { fwd(kFwdReg); });
-        tu.fwd = twv < tb ? kFwdReg : kFwdBlock;
-        ctx.tuned_fwd[N] = tu.fwd;
-        plane_ms += std::min(tb, twv);
-      } else {
-        plane_ms += timed([&] { fwd(tu.fwd); });
-      }
-      plane_ms += mid(tu.group, tu.depth, tu.poses);
-      if (need_inv) {
-        const float tb = timed([&] { inv(kInvBlock); });
-        const float tr = timed([&] { inv(kInvReg); });
-        tu.inv = tr < tb ? kInvReg : kInvBlock;
-        ctx.tuned_inv[N] = tu.inv;
-        plane_ms += std::min(tb, tr);
-      } else {
-        plane_ms += timed([&] { inv(tu.inv); });
-      }
-    }
-    if (need_col || (need_pipe && cols)) {
-      col_ms += timed([&] {
+    best += timed([&] {
+      hip_check(launch_inv_argmin(ctx.stream, N, tu.inv, d_meta, n, N - 2, ctx.w_T, d_keys, tw), "tune inverse");
+    });
+    if (col_ok) {
+      float ms = timed([&] {
         hip_check(launch_fwd_z(ctx.stream, N, sl, n, d_ligs, t.d_chan.as<int>(), t.d_wv.as<float>(),
                                t.d_wq.as<float>(), ctx.w_ag, t.astride, d_meta, t.cmax, t.boxmax,
                                t.max_chan_atoms, ctx.w_A, tw),
                   "tune column forward");
       });
-      auto midc = [&](int g) {
-        return timed([&] {
-          hip_check(launch_mid_kz(ctx.stream, N, sl, d_ligs, d_meta, n, g, ctx.w_A, t.cmax, t.boxmax,
-                                  prot.spec_kz.as<float2>(), ctx.w_T, invG, tw),
-                    "tune column mid");
-        });
-      };
-      if (need_col) {
-        col_ms += best_group(midc, tu.col_group);
-        ctx.tuned_col_group[ckey] = tu.col_group;
-      } else {
-        col_ms += midc(tu.col_group);
-      }
-      col_ms += timed([&] {
+      ms += timed([&] {
+        hip_check(launch_mid_kz(ctx.stream, N, sl, d_ligs, d_meta, n, tu.col_group, ctx.w_A, t.cmax, t.boxmax,
+                                prot.spec_kz.as<float2>(), ctx.w_T, invG, tw),
+                  "tune column mid");
+      });
+      ms += timed([&] {
         hip_check(launch_inv_z(ctx.stream, N, d_meta, n, ctx.w_T, d_keys, tw), "tune column inverse");
       });
+      if (ms < best) {
+        best = ms;
+        tu.pipe = kPipeColumns;
+      }
     }
-    if (need_pipe && atoms) {
-      atom_ms += timed([&] {
+    if (atoms_ok) {
+      float ms = timed([&] {
         hip_check(launch_mid_atoms(ctx.stream, N, sl, d_ligs, t.d_pad.as<int>(), t.d_wv.as<float>(),
                                    t.d_wq.as<float>(), ctx.w_ag, t.astride, d_meta, n, tu.atom_group,
                                    prot.spec_mf.as<float2>(), ctx.w_T, invG, tw, ctx.atom_products),
                   "tune atom mid");
       });
-      atom_ms += timed([&] {
+      ms += timed([&] {
         hip_check(launch_inv_z(ctx.stream, N, d_meta, n, ctx.w_T, d_keys, tw), "tune atom inverse");
       });
+      if (ms < best) tu.pipe = kPipeAtoms;
     }
-    if (need_pipe) {
-      tu.pipe = kPipePlanes;
-      float best = plane_ms;
-      if (cols && col_ms < best) {
-        best = col_ms;
-        tu.pipe = kPipeColumns;
-      }
-      if (atoms && atom_ms < best) {
-        best = atom_ms;
-        tu.pipe = kPipeAtoms;
-      }
-      ctx.tuned_pipe[N] = tu.pipe;
-    }
+    ctx.tuned_pipe[N] = tu.pipe;
   } catch (...) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);

@@ -231,22 +231,18 @@ struct Context {
   int mid_group = 0;              // poses per mid-stage workgroup; 0 = tuned
   int mid_depth = 0;              // mid-stage register ring depth with a fixed group; 0 = 2
   int mid_poses = 0;              // poses sharing each protein load in the mid stage with a fixed group; 0 = 1
-  int pipeline = -1;              // fused pipeline form (kPipePlanes, kPipeColumns, kPipeAtoms); -1 = tuned
+  int pipeline = -1;              // fused pipeline form (kPipePlanes, kPipeColumns, kPipeAtoms); -1 = chosen once per grid edge
   int overlap_z = 1;              // atom form: overlap each launch set's z-inverse stage with the next set
   int atom_products = 2;          // atom form products: kAtomF16x3 (exact 3-part FP16 splits), kAtomF16, kAtomF32
-  int fwd_variant = -1;           // forward plane stage form; -1 = tuned
-  int inv_variant = -1;           // inverse plane stage form; -1 = tuned
+  int fwd_variant = -1;           // forward plane stage form; -1 = by grid edge
+  int inv_variant = -1;           // inverse plane stage form; -1 = by grid edge
   bool use_graph = true;
   bool time_stages = false;
-  // Autotuner state.  The forward and inverse plane forms change FFT
-  // rounding, so each is chosen once per grid size and kept for the
-  // context's life (results then do not depend on how poses are batched);
-  // the mid group size only changes the schedule.
   size_t max_dyn_lds = 64 * 1024;
-  std::map<int, int> tuned_pipe;                     // N -> pipeline form
-  std::map<int, int> tuned_fwd;                      // N -> variant
-  std::map<int, int> tuned_inv;                      // N -> variant
-  std::map<std::array<int, 4>, int> tuned_col_group;   // (N, cmax, 0, 0) -> column form group
+  // The pipeline form taken, per grid edge: the forms round differently, so it
+  // is chosen once and kept for the context's life (results then do not depend
+  // on how poses are batched).
+  std::map<int, int> tuned_pipe;
   int last_fwd = -1, last_inv = -1, last_group = 0, last_depth = 0, last_poses = 0,
       last_pipe = -1;
   StageTimes stage_times;
@@ -293,9 +289,6 @@ void protein_build(Protein& p, int natom, const double* xyz, const double* charg
 // Largest job (in launch sets) captured as one hipGraph; larger jobs launch
 // eagerly.
 constexpr size_t kMaxGraphSets = 2048;
-// Plane-form schedules remembered per context; beyond this many the map drops
-// its smallest key before adding one.
-constexpr size_t kMaxTunedShapes = 256;
 
 // Builds and uploads the tables of a set of jobs (inputs resident in HBM).
 void prepare_search(Context& ctx, const Protein& prot, const std::vector<Job>& jobs, Prepared& t);

@@ -65,7 +65,9 @@ int cdk_context_destroy(cdk_context* ctx);
  * transform and whose mid stage runs the y and x transforms per kz plane;
  * 2 atom form at 64^3, 96^3 and 128^3, whose mid stage builds each channel's ligand
  * spectrum per kz plane from the atoms as a sum of outer products on the
- * matrix cores, with no forward stage; -1 = autotuned once per grid size),
+ * matrix cores, with no forward stage; -1 = once per grid edge: the atom
+ * form where it is supported if the first search's ligands have at most 84
+ * atoms, else the fastest on that search's first launch set),
  * "atom_products" (the atom form's products: 2 = FP16 matrix cores on
  * operands split exactly into three FP16 parts each (after power-of-two
  * scaling), the six partial products down to 2^-22 with FP32 accumulation:
@@ -76,9 +78,9 @@ int cdk_context_destroy(cdk_context* ctx);
  * mid stage, with two T2 buffers; 0 = one stream; default 1),
  * "fwd_variant" (forward
  * plane stage: 0 block-wide LDS Stockham FFTs, 1 register four-step FFTs,
- * -1 = autotuned once per grid size), "inv_variant" (inverse
+ * -1 = 0 at 32^3 and 48^3, 1 from 64^3), "inv_variant" (inverse
  * plane stage + argmin: 0 block-wide LDS FFTs per plane, 1 register FFTs over
- * 4 planes per workgroup, -1 = autotuned once per grid size), "use_graph",
+ * 4 planes per workgroup, -1 = as fwd_variant), "use_graph",
  * "time_stages". */
 int cdk_context_set_option(cdk_context* ctx, const char* key, int64_t value);
 /* Reads an option back; also "last_fwd_variant", "last_inv_variant",

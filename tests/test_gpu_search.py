@@ -629,3 +629,24 @@ def test_schedule_32_shares_protein_loads(ctx, n, poses):
     assert np.isfinite(E).any()
     assert np.array_equal(E.view(np.uint32), Ef.view(np.uint32)) and np.array_equal(idx, ixf)
     assert np.array_equal(mc.view(np.uint32), mcf.view(np.uint32))
+
+
+@pytest.mark.parametrize("n,box,natom,nquat,first", [(32, 16.0, 900, 20, dict(last_fwd_variant=0, last_inv_variant=0)),
+                                                     (64, 32.0, 3000, 200, dict(last_pipeline=2))])
+def test_forms_do_not_follow_the_first_call(n, box, natom, nquat, first):
+    """A new context whose first search is a small one (32^3, 20 poses; 64^3, a
+    one-atom ligand) takes the forms that a large search of an ordinary ligand
+    takes, not those that are fastest on that call."""
+    vals, radii, mid, ln = cdk.synth_protein(15, natom, box, n, 0.5)
+    c = cdk.Context(0)
+    prot = cdk.Protein(c, vals, radii, 0.5, mid, ln)
+    x, q, e, r = cdk.synth_ligand(841, 8 if n == 32 else 1)
+    lig = cdk.Ligand(prot, q, e, r)
+    quats = cdk.QuaternionUniformSampling(cdk.Rng(31), nquat)
+    say("first call %d^3" % n)
+    cdk.search(c, prot, lig, (x[None] * 0.5).astype(np.float32), quats)
+    got = {k: c.get_option(k) for k in first}
+    lig.close()
+    prot.close()
+    c.close()
+    assert got == first
