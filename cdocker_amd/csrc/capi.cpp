@@ -147,6 +147,11 @@ int cdk_context_set_option(cdk_context* ctx, const char* key, int64_t v) {
     if (k == "ws_budget_bytes") {
       require(v > 0, "budget must be positive");
       c.ws_budget = (size_t)v;
+    } else if (k == "scratch_keep_bytes") {
+      require(v >= 0, "scratch_keep_bytes must not be negative");
+      cdk::hip_check(hipSetDevice(c.device), "hipSetDevice");
+      c.scratch_keep = (size_t)v;
+      c.trim_scratch();
     } else if (k == "ref_batch") {
       require(v > 0 && v <= 100000, "ref_batch out of range");
       c.ref_batch = (int)v;
@@ -196,6 +201,8 @@ int cdk_context_get_option(cdk_context* ctx, const char* key, int64_t* value) {
     std::lock_guard<std::mutex> lk(c.mu);
     const std::string k(key);
     if (k == "ws_budget_bytes") *value = (int64_t)c.ws_budget;
+    else if (k == "scratch_keep_bytes") *value = (int64_t)c.scratch_keep;
+    else if (k == "scratch_bytes") *value = (int64_t)c.scratch_bytes();
     else if (k == "ref_batch") *value = c.ref_batch;
     else if (k == "fused_chunk") *value = c.fused_chunk;
     else if (k == "mid_group") *value = c.mid_group;

@@ -86,16 +86,37 @@ CallScratch::CallScratch(Context& c) : ctx_(c), exceptions_(std::uncaught_except
 
 CallScratch::~CallScratch() {
   if (std::uncaught_exceptions() > exceptions_) (void)hipStreamSynchronize(ctx_.stream);
-  if (ctx_.call_dev.cap > kKeepDev) {
-    (void)hipStreamSynchronize(ctx_.stream);
-    ctx_.call_dev.release();
+  ctx_.trim_call_arenas();
+}
+
+void Context::trim_call_arenas() {
+  const size_t keep = scratch_keep;
+  const bool dev_over = call_dev.cap > keep, host_over = call_host_cap > keep / 2;
+  if (dev_over || host_over) (void)hipStreamSynchronize(stream);
+  if (dev_over) call_dev.release();
+  if (host_over) {
+    (void)hipHostFree(call_host);
+    call_host = nullptr;
+    call_host_cap = 0;
   }
-  if (ctx_.call_host_cap > kKeepHost) {
-    (void)hipStreamSynchronize(ctx_.stream);
-    (void)hipHostFree(ctx_.call_host);
-    ctx_.call_host = nullptr;
-    ctx_.call_host_cap = 0;
-  }
+}
+
+bool Context::may_keep(const Prepared& t) const {
+  const size_t most = scratch_keep / 2;
+  return t.d_all.cap <= most && t.h_up_cap <= most && t.h_res_cap <= most;
+}
+
+void Context::trim_scratch() {
+  trim_call_arenas();
+  std::lock_guard<std::mutex> lock(idle_mu);
+  idle.erase(std::remove_if(idle.begin(), idle.end(), [&](const auto& t) { return !may_keep(*t); }), idle.end());
+}
+
+size_t Context::scratch_bytes() {
+  size_t n = call_dev.cap + call_host_cap;
+  std::lock_guard<std::mutex> lock(idle_mu);
+  for (const auto& t : idle) n += t->d_all.cap + t->h_up_cap + t->h_res_cap;
+  return n;
 }
 
 char* CallScratch::dev(size_t bytes) {
@@ -1230,11 +1251,8 @@ void run_search(Context& ctx, const Protein& prot, const Job& job, Engine engine
     }
   }
   t->prot = nullptr;
-  if (t->d_all.cap <= Context::kIdleBytes && t->h_up_cap <= Context::kIdleBytes &&
-      t->h_res_cap <= Context::kIdleBytes) {
-    std::lock_guard<std::mutex> lock(ctx.idle_mu);
-    if (ctx.idle.size() < Context::kIdleSearches) ctx.idle.push_back(std::move(t));
-  }
+  std::lock_guard<std::mutex> lock(ctx.idle_mu);
+  if (ctx.may_keep(*t) && ctx.idle.size() < Context::kIdleSearches) ctx.idle.push_back(std::move(t));
 }
 
 namespace {

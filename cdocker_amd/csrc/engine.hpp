@@ -3,8 +3,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <cstdint>
 #include <array>
+#include <atomic>
+#include <cstdint>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -58,13 +59,13 @@ struct Context;
 
 // One call's use of its context's scratch memory (the context lock held for
 // the object's life): a device arena and a pinned host arena that grow to what
-// a call needs and stay with the context for the next, up to kKeepDev and
-// kKeepHost bytes; a call that needed more gives the excess back when it ends.
+// a call needs and stay with the context for the next, up to its scratch_keep
+// bytes and half as many; a call that needed more gives its arena back when it
+// ends.
 // A call that ends by an exception waits for the stream first, so nothing
 // queued still reads or writes the arenas.
 class CallScratch {
  public:
-  static constexpr size_t kKeepDev = 128ull << 20, kKeepHost = 64ull << 20;
   explicit CallScratch(Context& c);
   ~CallScratch();
   CallScratch(const CallScratch&) = delete;
@@ -266,16 +267,25 @@ struct Context {
   void* call_host = nullptr;
   size_t call_host_cap = 0;
   std::vector<hipEvent_t> call_events;
+  // Most bytes the device arena keeps between calls; the host arena and each
+  // buffer of the idle tables keep half as many.
+  std::atomic<size_t> scratch_keep{128ull << 20};
   // Tables of finished cdk_search calls, kept for the next ones: at most
-  // kIdleSearches of at most kIdleBytes each.  Every call takes one for
-  // itself, so calls of several threads never share one.
-  static constexpr size_t kIdleSearches = 2, kIdleBytes = 64ull << 20;
+  // kIdleSearches of them.  Every call takes one for itself, so calls of
+  // several threads never share one.
+  static constexpr size_t kIdleSearches = 2;
   std::mutex idle_mu;
   std::vector<std::unique_ptr<Prepared>> idle;
 
   explicit Context(int dev);
   ~Context();
   const float2* twiddle(int N);
+  // Device and pinned host bytes kept for the synchronous calls, and those
+  // above scratch_keep given back (context lock held).
+  size_t scratch_bytes();
+  void trim_scratch();
+  void trim_call_arenas();
+  bool may_keep(const Prepared& t) const;
 };
 
 void protein_upload(Protein& p, int nch, int N, float h, const float* mid, const float* len, const float* radii,

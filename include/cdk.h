@@ -53,7 +53,12 @@ int cdk_version(void);
  * TranRotaConfSearchNoMini.cu:156-252. */
 int cdk_context_create(int device, cdk_context** out);
 int cdk_context_destroy(cdk_context* ctx);
-/* Options: "ws_budget_bytes", "ref_batch" (B, default 50 as NoMini:208),
+/* Options: "ws_budget_bytes", "scratch_keep_bytes" (device bytes of the
+ * synchronous calls' scratch kept between calls, default 128 MB; pinned host
+ * scratch and each table buffer of up to two finished searches: half as many;
+ * a call that needs more takes it and gives it back when it ends; setting a
+ * smaller value gives back what is above it at once, 0 keeps nothing),
+ * "ref_batch" (B, default 50 as NoMini:208),
  * "fused_chunk" (poses per fused launch set, 0 = from budget), "mid_group"
  * (poses per mid-stage workgroup, 0 = by the size of the launch),
  * "mid_depth" (register buffers in the mid stage's (pose, channel) ring when
@@ -89,7 +94,9 @@ int cdk_context_set_option(cdk_context* ctx, const char* key, int64_t value);
  * device's dynamic LDS limit per workgroup, bytes) and "workspace_bytes"
  * (device bytes of the fused engine's launch-set working arrays: one pool,
  * carved per search; never above "ws_budget_bytes" unless "fused_chunk"
- * forces larger launch sets).  No reference counterpart. */
+ * forces larger launch sets), "scratch_bytes" (device and pinned host bytes
+ * now kept under "scratch_keep_bytes"; not part of "workspace_bytes").  No
+ * reference counterpart. */
 int cdk_context_get_option(cdk_context* ctx, const char* key, int64_t* value);
 /* Per-stage device time (HIP events on the context stream) accumulated while
  * "time_stages" is on: ms[8], launches[8].  Stage ids: reference engine

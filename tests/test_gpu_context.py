@@ -1,0 +1,63 @@
+"""What a context keeps between calls: scratch memory, idle search tables and
+captured graphs never change a result, whichever call came before."""
+import numpy as np
+import pytest
+
+import cdocker_amd as cdk
+from cdocker_amd import workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print("[gpu]", *a, flush=True)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = cdk.Context(0)
+    yield c
+    c.close()
+
+
+def make(ctx, n=48, natom_protein=500):
+    vals, radii, mid, ln = cdk.synth_protein(15, natom_protein, 0.5 * n, n, 0.5)
+    return cdk.Protein(ctx, vals, radii, 0.5, mid, ln)
+
+
+def bits(*arrays):
+    return [np.ascontiguousarray(a).view(np.uint8).tobytes() for a in arrays if a is not None]
+
+
+def test_scratch_is_counted_and_given_back(ctx):
+    """The bytes kept for the next calls can be read, are given back when the
+    limit is lowered, stay given back while it is 0, and do not change results."""
+    say("scratch")
+    prot = make(ctx)
+    x, q, e, r = cdk.synth_ligand(3, 12)
+    lig = cdk.Ligand(prot, q, e, r)
+    quats = cdk.QuaternionUniformSampling(cdk.Rng(5), 40)
+    rot, mv, ex = workloads.chain_topology(12)
+    poses = x[None].astype(np.float64) + np.linspace(9, 12, 30)[:, None, None]
+
+    def calls():
+        return bits(*cdk.search(ctx, prot, lig, x[None], quats), *cdk.rescore_poses(prot, lig, poses, want_grad=True),
+                    *cdk.refine_poses(prot, lig, poses, steps=4),
+                    *cdk.generate_conformers(ctx, x, rot, mv, ex, 60, 3, 0.6), prot.grids())
+
+    assert ctx.get_option("scratch_keep_bytes") == 128 << 20
+    first = calls()
+    kept = ctx.get_option("scratch_bytes")
+    assert 0 < kept <= 3 * (128 << 20)
+    try:
+        ctx.set_option("scratch_keep_bytes", 0)
+        assert ctx.get_option("scratch_bytes") == 0
+        assert calls() == first
+        assert ctx.get_option("scratch_bytes") == 0
+        with pytest.raises(cdk.CdkError):
+            ctx.set_option("scratch_keep_bytes", -1)
+    finally:
+        ctx.set_option("scratch_keep_bytes", 128 << 20)
+    assert calls() == first and ctx.get_option("scratch_bytes") > 0
+    lig.close()
+    prot.close()
