@@ -1350,6 +1350,9 @@ void refine_poses(Context& ctx, const Protein& prot, const Ligand& lig, int npos
   }
 }
 
+// Device bytes of a set of conformer trials (512 atoms: 4 096 trials, 101 MB).
+constexpr size_t kConformerBytes = 64ull << 20;
+
 int generate_conformers(Context& ctx, int natom, const double* coords, int nrotor, const int* rotors,
                         const unsigned char* moving, const unsigned char* exclude, int ntrial, uint64_t seed,
                         double clash_dist, int max_keep, double* out, int* trial_index) {
@@ -1364,12 +1367,15 @@ int generate_conformers(Context& ctx, int natom, const double* coords, int nroto
   // Trials run a set at a time and stop once enough have passed: the kept
   // ones are the first max_keep in trial order, so later trials cannot
   // matter.  A first set of 4 096 (four wavefronts per SIMD) takes hardly
-  // longer than one of a few; the next sets follow the share that passed.
+  // longer than one of a few; the next sets follow the share that passed.  No
+  // set is larger than kConformerBytes allow for its trials' coordinates and
+  // the kept ones' copies, so a call that keeps most of many trials needs no
+  // more memory than another.
   int kept = 0, done = 0;
-  int set = std::min(ntrial, std::max(4096, max_keep));
-  // no later set is larger than this
-  const size_t cap = (size_t)std::min<long long>(ntrial, std::max(1 << 16, set));
+  const size_t most = std::max<size_t>(4096, kConformerBytes / (2 * std::max<size_t>(per, 1) * sizeof(double)));
+  const size_t cap = std::min({(size_t)ntrial, most, (size_t)1 << 16});
   const size_t keep = std::min<size_t>(max_keep, cap);
+  int set = (int)std::min(cap, std::max<size_t>(4096, max_keep));
   CallScratch scratch(ctx);
   Layout in, l;
   const size_t o_x = in.add(per * sizeof(double)), o_rot = in.add((size_t)nrotor * 4 * sizeof(int));

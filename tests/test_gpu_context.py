@@ -61,3 +61,25 @@ def test_scratch_is_counted_and_given_back(ctx):
     assert calls() == first and ctx.get_option("scratch_bytes") > 0
     lig.close()
     prot.close()
+
+
+def test_conformers_that_all_pass_need_no_more_memory(ctx):
+    """A call that keeps every one of many trials runs them in sets of bounded
+    memory: the scratch it leaves is below the coordinates it returns, trial
+    numbers are complete, and conformers across sets are those of a call for
+    fewer (trials depend on their number alone)."""
+    natom, ntrial = 24, 150000
+    x, q, e, r = cdk.synth_ligand(77, natom)
+    rot, mv, ex = workloads.chain_topology(natom)
+    ctx.set_option("scratch_keep_bytes", 0)
+    try:
+        ctx.set_option("scratch_keep_bytes", 1 << 40)
+        say("conformers, all kept")
+        conf, trial = cdk.generate_conformers(ctx, x, rot, mv, ex, ntrial, 9, 1e-6)
+        used = ctx.get_option("scratch_bytes")
+    finally:
+        ctx.set_option("scratch_keep_bytes", 128 << 20)
+    assert np.array_equal(trial, np.arange(ntrial))
+    assert used < ntrial * natom * 24 + (24 << 20)
+    few, t = cdk.generate_conformers(ctx, x, rot, mv, ex, 70000, 9, 1e-6, max_keep=69990)
+    assert np.array_equal(t, np.arange(69990)) and np.array_equal(few, conf[:69990])
