@@ -1267,34 +1267,50 @@ void atom_channels(const Protein& prot, const Ligand& lig, std::vector<int>& pch
   (void)prot;
 }
 
-// Poses whose coordinates (and gradients) go through the pinned arena at a
-// time, and the parts of that arena: the ligand's channels and weights, then
-// the poses' coordinates and results.  The kernels read and write them in
-// place over the host link.
+// Poses go through the pinned arena in pieces, two slots in turn, so the host
+// copies one piece in and another out while the kernel works on a third; the
+// kernels read and write the slots in place over the host link.  A call within
+// one piece has one slot.  Measured, one slot of 32 MB -> two of 4 MB, 40 atoms:
+// 200 000 poses rescored 10.0 -> 7.1 ms, with the gradient 25.7 -> 20.8, 40 000
+// refined for 50 steps 8.5 -> 7.5.  Two of 1 / 2 / 8 MB: 7.9 / 7.4 / 7.0 ms, 18.3
+// / 17.2 / 20.9, 8.6 / 7.6 / 7.2; small ones leave large poses' kernels short
+// (500 poses of 300 atoms refined 0.97 / 0.67 / 0.64 ms, 4 MB 0.61).
 struct PoseStage {
-  int per = 0;  // poses per piece
-  int *pch = nullptr, *inside = nullptr;
+  int per = 0;    // poses per piece
+  int slots = 1;
+  // the ligand's channels and weights, then per slot the poses' coordinates
+  // and results
+  int* pch = nullptr;
   float *wv = nullptr, *wq = nullptr;
-  double *x = nullptr, *g = nullptr, *e = nullptr;
+  int* inside[2] = {};
+  double *x[2] = {}, *g[2] = {}, *e[2] = {};
 };
-constexpr size_t kPoseStageBytes = 32ull << 20;
+constexpr size_t kPosePieceBytes = 4ull << 20;
 
 PoseStage stage_poses(CallScratch& scratch, const Protein& prot, const Ligand& lig, int npose, bool grad) {
   const size_t na = (size_t)lig.natom, pose = na * 3 * sizeof(double);
   PoseStage s;
-  s.per = (int)std::max<size_t>(1, std::min<size_t>((size_t)npose, kPoseStageBytes / ((grad ? 2 : 1) * pose + 16)));
+  s.per = (int)std::max<size_t>(1, std::min<size_t>((size_t)npose, kPosePieceBytes / ((grad ? 2 : 1) * pose + 16)));
+  s.slots = s.per < npose ? 2 : 1;
   Layout l;
   const size_t o_pch = l.add(na * sizeof(int)), o_wv = l.add(na * sizeof(float)), o_wq = l.add(na * sizeof(float));
-  const size_t o_e = l.add(s.per * sizeof(double)), o_in = l.add(s.per * sizeof(int));
-  const size_t o_x = l.add(s.per * pose), o_g = grad ? l.add(s.per * pose) : 0;
+  size_t o_e[2], o_in[2], o_x[2], o_g[2];
+  for (int i = 0; i < s.slots; ++i) {
+    o_e[i] = l.add(s.per * sizeof(double));
+    o_in[i] = l.add(s.per * sizeof(int));
+    o_x[i] = l.add(s.per * pose);
+    o_g[i] = grad ? l.add(s.per * pose) : 0;
+  }
   char* h = scratch.host(l.end);
   s.pch = reinterpret_cast<int*>(h + o_pch);
   s.wv = reinterpret_cast<float*>(h + o_wv);
   s.wq = reinterpret_cast<float*>(h + o_wq);
-  s.e = reinterpret_cast<double*>(h + o_e);
-  s.inside = reinterpret_cast<int*>(h + o_in);
-  s.x = reinterpret_cast<double*>(h + o_x);
-  if (grad) s.g = reinterpret_cast<double*>(h + o_g);
+  for (int i = 0; i < s.slots; ++i) {
+    s.e[i] = reinterpret_cast<double*>(h + o_e[i]);
+    s.inside[i] = reinterpret_cast<int*>(h + o_in[i]);
+    s.x[i] = reinterpret_cast<double*>(h + o_x[i]);
+    if (grad) s.g[i] = reinterpret_cast<double*>(h + o_g[i]);
+  }
   std::vector<int> pch;
   atom_channels(prot, lig, pch);
   for (int a = 0; a < lig.natom; ++a) {
@@ -1303,6 +1319,32 @@ PoseStage stage_poses(CallScratch& scratch, const Protein& prot, const Ligand& l
     s.wq[a] = lig.charge[a];
   }
   return s;
+}
+
+// run(slot, n) for the pieces of npose poses, coords copied in before and
+// done(slot, first, n) called after each.
+template <class Run, class Done>
+void for_pieces(Context& ctx, const PoseStage& w, int npose, size_t per_pose, const double* coords, Run&& run,
+                Done&& done) {
+  slot_events(ctx);
+  int before = 0, first = 0;  // the piece before: its poses and their first
+  for (int p0 = 0, i = 0; p0 < npose; ++i) {
+    const int n = std::min(w.per, npose - p0), slot = i & 1;
+    std::memcpy(w.x[slot], coords + p0 * per_pose, n * per_pose * sizeof(double));
+    run(slot, n);
+    if (p0 + n < npose) hip_check(hipEventRecord(ctx.call_events[slot], ctx.stream), "hipEventRecord");
+    if (i > 0) {
+      hip_check(hipEventSynchronize(ctx.call_events[slot ^ 1]), "pose piece");
+      done(slot ^ 1, first, before);
+    }
+    first = p0;
+    before = n;
+    p0 += n;
+    if (p0 == npose) {
+      hip_check(hipStreamSynchronize(ctx.stream), "pose pieces");
+      done(slot, first, before);
+    }
+  }
 }
 
 }  // namespace
@@ -1316,17 +1358,18 @@ void rescore_poses(Context& ctx, const Protein& prot, const Ligand& lig, int npo
   const PoseStage w = stage_poses(scratch, prot, lig, npose, grad != nullptr);
   const double gmin[3] = {prot.grid_min(0), prot.grid_min(1), prot.grid_min(2)};
   const size_t per = (size_t)lig.natom * 3;
-  for (int p0 = 0; p0 < npose; p0 += w.per) {
-    const int n = std::min(w.per, npose - p0);
-    std::memcpy(w.x, coords + p0 * per, n * per * sizeof(double));
-    hip_check(launch_rescore(ctx.stream, n, lig.natom, w.x, w.pch, w.wv, w.wq, prot.grid.as<float>(), prot.N,
-                             prot.nch - 1, gmin, (double)prot.h, w.e, w.g, w.inside),
-              "rescore");
-    hip_check(hipStreamSynchronize(ctx.stream), "rescore sync");
-    std::memcpy(energy + p0, w.e, n * sizeof(double));
-    if (grad) std::memcpy(grad + p0 * per, w.g, n * per * sizeof(double));
-    if (inside) std::memcpy(inside + p0, w.inside, n * sizeof(int));
-  }
+  for_pieces(
+      ctx, w, npose, per, coords,
+      [&](int slot, int n) {
+        hip_check(launch_rescore(ctx.stream, n, lig.natom, w.x[slot], w.pch, w.wv, w.wq, prot.grid.as<float>(), prot.N,
+                                 prot.nch - 1, gmin, (double)prot.h, w.e[slot], w.g[slot], w.inside[slot]),
+                  "rescore");
+      },
+      [&](int slot, int p0, int n) {
+        std::memcpy(energy + p0, w.e[slot], n * sizeof(double));
+        if (grad) std::memcpy(grad + p0 * per, w.g[slot], n * per * sizeof(double));
+        if (inside) std::memcpy(inside + p0, w.inside[slot], n * sizeof(int));
+      });
 }
 
 void refine_poses(Context& ctx, const Protein& prot, const Ligand& lig, int npose, double* coords, int steps,
@@ -1338,16 +1381,17 @@ void refine_poses(Context& ctx, const Protein& prot, const Ligand& lig, int npos
   const PoseStage w = stage_poses(scratch, prot, lig, npose, false);
   const double gmin[3] = {prot.grid_min(0), prot.grid_min(1), prot.grid_min(2)};
   const size_t per = (size_t)lig.natom * 3;
-  for (int p0 = 0; p0 < npose; p0 += w.per) {
-    const int n = std::min(w.per, npose - p0);
-    std::memcpy(w.x, coords + p0 * per, n * per * sizeof(double));
-    hip_check(launch_refine(ctx.stream, n, lig.natom, w.x, w.pch, w.wv, w.wq, prot.grid.as<float>(), prot.N,
-                            prot.nch - 1, gmin, (double)prot.h, steps, penalty, w.e),
-              "refine");
-    hip_check(hipStreamSynchronize(ctx.stream), "refine sync");
-    std::memcpy(coords + p0 * per, w.x, n * per * sizeof(double));
-    std::memcpy(energy + p0, w.e, n * sizeof(double));
-  }
+  for_pieces(
+      ctx, w, npose, per, coords,
+      [&](int slot, int n) {
+        hip_check(launch_refine(ctx.stream, n, lig.natom, w.x[slot], w.pch, w.wv, w.wq, prot.grid.as<float>(), prot.N,
+                                prot.nch - 1, gmin, (double)prot.h, steps, penalty, w.e[slot]),
+                  "refine");
+      },
+      [&](int slot, int p0, int n) {
+        std::memcpy(coords + p0 * per, w.x[slot], n * per * sizeof(double));
+        std::memcpy(energy + p0, w.e[slot], n * sizeof(double));
+      });
 }
 
 // Device bytes of a set of conformer trials (512 atoms: 4 096 trials, 101 MB).

@@ -83,3 +83,33 @@ def test_conformers_that_all_pass_need_no_more_memory(ctx):
     assert used < ntrial * natom * 24 + (24 << 20)
     few, t = cdk.generate_conformers(ctx, x, rot, mv, ex, 70000, 9, 1e-6, max_keep=69990)
     assert np.array_equal(t, np.arange(69990)) and np.array_equal(few, conf[:69990])
+
+
+@pytest.mark.parametrize("natom,npose", [(40, 4346), (40, 9000), (1, 120000), (300, 601), (512, 342)])
+def test_poses_in_pieces(ctx, natom, npose):
+    """Rescoring and refinement of more poses than one piece of the pinned
+    memory holds (two and more pieces, whole and odd remainders): bit for bit
+    the results of the same poses in calls of their own."""
+    say("pieces natom=%d npose=%d" % (natom, npose))
+    prot = make(ctx)
+    rs = np.random.default_rng(natom)
+    _, q, e, r = cdk.synth_ligand(19, natom)
+    lig = cdk.Ligand(prot, q, e, r)
+    x = rs.normal(0, 2.0, (natom, 3))
+    poses = x[None] + rs.uniform(7, 16, (npose, 1, 3))
+    cuts = np.unique([0, 50, npose // 4, npose // 2, 3 * npose // 4, npose - 1, npose])
+    parts = list(zip(cuts, cuts[1:]))
+    for grad in (True, False):
+        E, g, ins = cdk.rescore_poses(prot, lig, poses, want_grad=grad)
+        assert np.isfinite(E).all() and len(np.unique(E)) > 100
+        for a, b in parts:
+            for lo, hi in ((a, min(a + 300, b)), (max(a, b - 300), b)):
+                Es, gs, inss = cdk.rescore_poses(prot, lig, poses[lo:hi], want_grad=grad)
+                assert bits(Es, gs, inss) == bits(E[lo:hi], g[lo:hi] if grad else None, ins[lo:hi]), (lo, hi)
+    X, E = cdk.refine_poses(prot, lig, poses, steps=2)
+    for a, b in parts:
+        for lo, hi in ((a, min(a + 200, b)), (max(a, b - 200), b)):
+            Xs, Es = cdk.refine_poses(prot, lig, poses[lo:hi], steps=2)
+            assert bits(Xs, Es) == bits(X[lo:hi], E[lo:hi]), (lo, hi)
+    lig.close()
+    prot.close()
