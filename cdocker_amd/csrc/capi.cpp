@@ -313,7 +313,8 @@ int cdk_protein_spectrum(cdk_protein* p, int channel, float* out) {
 int cdk_protein_bytes(cdk_protein* p, int64_t* bytes) {
   return guard([&] {
     require(p && bytes, "NULL argument");
-    *bytes = (int64_t)p->p.all.cap;
+    *bytes = 0;
+    for (const cdk::DevBuf& m : p->p.mem) *bytes += (int64_t)m.cap;
   });
 }
 

@@ -106,7 +106,7 @@ struct Protein {
   float mid[3] = {0, 0, 0};
   float len[3] = {0, 0, 0};
   std::vector<float> radii;  // nch - 1 probe radii
-  DevBuf all;                // one allocation: the grids and every copy of the spectra
+  DevBuf mem[5];             // the memory of the arrays below, one block or one each
   DevView grid;              // float [nch][G]
   DevView spec;              // float2 [nch][H]
   DevView spec_lb;           // the same spectra in the fused engine's line-blocked layout

@@ -113,3 +113,31 @@ def test_poses_in_pieces(ctx, natom, npose):
             assert bits(Xs, Es) == bits(X[lo:hi], E[lo:hi]), (lo, hi)
     lig.close()
     prot.close()
+
+
+@pytest.mark.parametrize("nch", [2, 15, 16])
+def test_protein_memory_by_size(ctx, nch):
+    """32^3 proteins on both sides of the size from which one allocation holds
+    every array (16 channels): grids read back bit for bit, spectra are the
+    grids' transforms, and the fused engine (which reads another copy of the
+    spectra) agrees with the reference dataflow."""
+    say("protein channels", nch)
+    rs = np.random.default_rng(nch)
+    n = 32
+    v = rs.normal(0, 1, (nch, n, n, n)).astype(np.float32)
+    radii = np.linspace(1.0, 2.2, nch - 1).astype(np.float32)
+    prot = cdk.Protein(ctx, v, radii, 0.5)
+    H = nch * n * n * (n // 2 + 1) * 8
+    assert v.nbytes + 2 * H <= prot.device_bytes() <= v.nbytes + 2 * H + 5 * 256
+    assert bits(prot.grids()) == bits(v)
+    for c in (0, nch - 1):
+        ref = np.fft.rfftn(v[c].astype(np.float64))
+        assert np.abs(prot.spectrum(c) - ref).max() <= 1e-5 * np.abs(ref).max()
+    x, q, e, r = cdk.synth_ligand(23, 7)
+    lig = cdk.Ligand(prot, q, e, r)
+    quats = cdk.QuaternionUniformSampling(cdk.Rng(7), 9)
+    E, idx, _ = cdk.search(ctx, prot, lig, x[None], quats)
+    R, ridx, _ = cdk.search(ctx, prot, lig, x[None], quats, engine=cdk.ENGINE_REFERENCE)
+    assert np.isfinite(R).all() and np.abs(E - R).max() <= 1e-4 * np.abs(R).max()
+    lig.close()
+    prot.close()
