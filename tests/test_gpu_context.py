@@ -141,3 +141,63 @@ def test_protein_memory_by_size(ctx, nch):
     assert np.isfinite(R).all() and np.abs(E - R).max() <= 1e-4 * np.abs(R).max()
     lig.close()
     prot.close()
+
+
+@pytest.mark.parametrize("n,pipeline,chunk", [(64, 2, 0), (64, 2, 7), (64, 1, 16), (64, 0, 16), (48, 0, 9), (96, 2, 11)])
+@pytest.mark.parametrize("overlap", [0, 1])
+def test_batch_graph_capture_and_replays(ctx, n, pipeline, chunk, overlap):
+    """One Batch run again and again: launched eagerly, captured, then replayed,
+    with eager searches on the same context between the runs, and captured anew
+    after the schedule changes, the working memory moves or a job is added.
+    Every run has the bits of a Batch that never uses a graph."""
+    say("graph n=%d pipeline=%d chunk=%d overlap=%d" % (n, pipeline, chunk, overlap))
+    prot = make(ctx, n)
+    jobs = []
+    for i in range(4):
+        x, q, e, r = cdk.synth_ligand(40 + i, 9 + 5 * i)
+        jobs.append((cdk.Ligand(prot, q, e, r), x[None], cdk.QuaternionUniformSampling(cdk.Rng(50 + i), 11)))
+
+    def eager(k):
+        ctx.set_option("use_graph", 0)
+        b = cdk.Batch(ctx, prot)
+        for j in jobs[:k]:
+            b.add(*j)
+        out = []
+        for _ in range(2):
+            b.run()
+            out.append([bits(*b.results(i)) for i in range(k)])
+        b.close()
+        ctx.set_option("use_graph", 1)
+        assert out[0] == out[1]
+        return out[0]
+
+    try:
+        ctx.set_option("overlap_z", overlap)
+        ctx.set_option("pipeline", pipeline)
+        ctx.set_option("fused_chunk", chunk)
+        want = {k: eager(k) for k in (3, 4)}
+        b = cdk.Batch(ctx, prot)
+        for j in jobs[:3]:
+            b.add(*j)
+        for run in range(9):
+            if run == 4:
+                ctx.set_option("mid_group", 3)  # captured anew
+            if run == 6:
+                ctx.set_option("mid_group", 0)
+                ctx.set_option("fused_chunk", 40)
+                cdk.search(ctx, prot, *jobs[3])  # the working memory grows
+                ctx.set_option("fused_chunk", chunk)
+            b.run()
+            assert [bits(*b.results(i)) for i in range(3)] == want[3], run
+            cdk.search(ctx, prot, *jobs[run % 4])
+        b.add(*jobs[3])
+        for run in range(4):
+            b.run()
+            assert [bits(*b.results(i)) for i in range(4)] == want[4], run
+        b.close()
+    finally:
+        for k, v in (("overlap_z", 1), ("pipeline", -1), ("fused_chunk", 0), ("mid_group", 0), ("use_graph", 1)):
+            ctx.set_option(k, v)
+        for j in jobs:
+            j[0].close()
+        prot.close()
