@@ -1,5 +1,7 @@
 """What a context keeps between calls: scratch memory, idle search tables and
 captured graphs never change a result, whichever call came before."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -201,3 +203,81 @@ def test_batch_graph_capture_and_replays(ctx, n, pipeline, chunk, overlap):
         for j in jobs:
             j[0].close()
         prot.close()
+
+
+def test_searches_of_several_threads(ctx):
+    """Threads that search, rescore and make conformers on one context at once
+    get what each gets alone: no two calls share kept tables or scratch."""
+    say("threads")
+    prots = {n: make(ctx, n) for n in (48, 64)}
+    rot, mv, ex = workloads.chain_topology(14)
+
+    def call(k):
+        prot = prots[(48, 64)[k % 2]]
+        x, q, e, r = cdk.synth_ligand(60 + k, 6 + 2 * k)
+        lig = cdk.Ligand(prot, q, e, r)
+        quats = cdk.QuaternionUniformSampling(cdk.Rng(70 + k), 5 + 9 * k)
+        out = bits(*cdk.search(ctx, prot, lig, x[None], quats))
+        poses = x[None].astype(np.float64) + np.linspace(9, 12, 20 + k)[:, None, None]
+        out += bits(*cdk.rescore_poses(prot, lig, poses, want_grad=True))
+        xc = cdk.synth_ligand(80 + k, 14)[0]
+        out += bits(*cdk.generate_conformers(ctx, xc, rot, mv, ex, 200, k, 0.6))
+        lig.close()
+        return out
+
+    for k in (0, 1):
+        call(k)  # the forms are chosen
+    want = [call(k) for k in range(8)]
+    got, errors = [[] for _ in range(8)], []
+
+    def work(k):
+        try:
+            for _ in range(6):
+                got[k].append(call(k))
+        except Exception as e:  # noqa: BLE001 - reported below
+            errors.append((k, e))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for k in range(8):
+        assert len(got[k]) == 6 and all(g == want[k] for g in got[k]), k
+    for p in prots.values():
+        p.close()
+
+
+def test_calls_after_calls_that_failed(ctx):
+    """A call that is refused, before or after its tables are built, leaves
+    nothing behind: the next calls have the results of a fresh context."""
+    say("failed calls")
+    prot = make(ctx)
+    x, q, e, r = cdk.synth_ligand(5, 11)
+    lig = cdk.Ligand(prot, q, e, r)
+    quats = cdk.QuaternionUniformSampling(cdk.Rng(9), 33)
+    rot, mv, ex = workloads.chain_topology(11)
+    poses = x[None].astype(np.float64) + np.linspace(9, 12, 12)[:, None, None]
+
+    def calls():
+        return bits(*cdk.search(ctx, prot, lig, x[None], quats), *cdk.refine_poses(prot, lig, poses, steps=3),
+                    *cdk.generate_conformers(ctx, x, rot, mv, ex, 50, 3, 0.6))
+
+    want = calls()
+    bad_quats = quats.copy()
+    bad_quats[-1, 2] = np.nan
+    bad_x = np.repeat(x[None], 2, 0)
+    bad_x[1, -1, 0] = np.inf
+    bad_rot = rot.copy()
+    bad_rot[-1, 3] = 99
+    for refused in (lambda: cdk.search(ctx, prot, lig, x[None], bad_quats),
+                    lambda: cdk.search(ctx, prot, lig, bad_x, quats),
+                    lambda: cdk.generate_conformers(ctx, x, bad_rot, mv, ex, 50, 3, 0.6),
+                    lambda: cdk.Protein(ctx, np.zeros((1, 48, 48, 48)), [1.0], 0.5),
+                    lambda: cdk.Protein(ctx, np.zeros((3, 40, 40, 40)), [1.0, 1.5], 0.5)):
+        with pytest.raises(cdk.CdkError):
+            refused()
+        assert calls() == want
+    lig.close()
+    prot.close()
