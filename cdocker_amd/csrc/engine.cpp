@@ -1169,7 +1169,6 @@ void decode_results(Prepared& t) {
 // Runs t's launch sequence to its end (context lock held).
 void run_prepared(Context& ctx, Prepared& t, Engine engine, bool use_graph) {
   EventTimer timer(ctx);
-  t.own_staging = false;
   enqueue_search(ctx, t, engine, use_graph, timer);
   hip_check(hipStreamSynchronize(ctx.stream), "search sync");
   t.h_up_busy = false;
@@ -1195,7 +1194,6 @@ void submit_search(Context& ctx, Prepared& t) {
   if (!t.prot) throw Error(kErrInvalid, "search not built");
   if (!t.start) hip_check(hipEventCreate(&t.start), "hipEventCreate");
   if (!t.done) hip_check(hipEventCreate(&t.done), "hipEventCreate");
-  t.own_staging = true;
   upload_tables(ctx, t);
   if (t.slots.empty()) {
     hip_check(hipEventRecord(t.start, ctx.stream), "hipEventRecord");

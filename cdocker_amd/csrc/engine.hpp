@@ -197,16 +197,14 @@ struct Prepared {
   int graph_group = 0, graph_fwd = -1, graph_inv = -1, graph_depth = 0, graph_poses = 0, graph_pipe = -1,
       graph_products = -1, graph_overlap = -1;
   std::vector<PoseResults> results;
-  // Pipelined callers (the server): the tables are uploaded from, and the
-  // results copied into, this table's own pinned staging, and `done` marks
-  // the end of its launch sequence on the context stream (`start` the first
-  // launch), so the host can build the next table while this one runs.
-  bool own_staging = false;
   void* h_up = nullptr;  // pinned staging of the tables' upload
   size_t h_up_cap = 0;
   bool h_up_busy = false;  // its last upload may still be queued
-  void* h_res = nullptr;   // own pinned staging of the results
+  void* h_res = nullptr;   // pinned staging of the results
   size_t h_res_cap = 0;
+  // Pipelined callers (the server): `done` marks the end of the launch
+  // sequence on the context stream (`start` the first launch), so the host can
+  // build the next table while this one runs.
   hipEvent_t start = nullptr, done = nullptr;
   Prepared() = default;
   Prepared(const Prepared&) = delete;
@@ -308,8 +306,8 @@ void execute_search(Context& ctx, Prepared& t, Engine engine, bool use_graph);
 // The same in pipelined pieces: build_search fills t's host tables (no
 // device work, no lock); submit_search uploads them and enqueues the fused
 // launch sequence and the result copies on the context stream without
-// waiting (t.own_staging is set; t's host tables must stay unchanged until
-// finish_search); finish_search waits for t's sequence and decodes
+// waiting (t's host tables must stay unchanged until finish_search);
+// finish_search waits for t's sequence and decodes
 // t.results.  Successive submissions run in stream order.
 void build_search(const Protein& prot, const std::vector<Job>& jobs, Prepared& t);
 void submit_search(Context& ctx, Prepared& t);

@@ -706,6 +706,13 @@ __device__ __forceinline__ void fwd_plane_rows(int x, const SpreadAtom* __restri
   __syncthreads();
 }
 
+// Its LDS scratch (float2): a slice per wavefront for the transforms of eight
+// lanes a line; those of four need none, only line 0's split does (wavefront 0).
+template <int N>
+constexpr int fwd_reg_scratch() {
+  return RegShape<N>::L == 8 ? 4 * RegShape<N>::SLICE : N;
+}
+
 template <class P>
 __global__ __launch_bounds__(kBlock) void k_fwd_planes_reg(const PoseSlot* __restrict__ slots,
                                                            const LigandDesc* __restrict__ ligs,
@@ -719,7 +726,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_planes_reg(const PoseSlot* __res
   using RS_ = RegShape<N>;
   constexpr int L = RS_::L, V = RS_::V, LPW = RS_::LPW, RSTR = FwdRegShape<N>::RSTR;
   constexpr bool TW_LDS = V >= 16;  // long lines: twiddles from LDS, registers to the data
-  __shared__ float2 sbuf[4][RS_::SLICE];
+  __shared__ float2 sbuf[fwd_reg_scratch<N>()];
   __shared__ float2 stw[TW_LDS ? L * V : 1];
   extern __shared__ double dyn[];  // [natom_lds] SpreadAtom, then the tile [npmax][RSTR]
   const int c = blockIdx.x, s = blockIdx.y;
@@ -750,7 +757,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_planes_reg(const PoseSlot* __res
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int ln = lane % LPW, n2 = lane / LPW;
-  float2* tr = sbuf[wave];
+  float2* tr = sbuf + (L == 8 ? wave * RS_::SLICE : 0);
   float2 twr[TW_LDS ? 1 : V];
   if constexpr (TW_LDS) {
     for (int t = threadIdx.x; t < L * V; t += blockDim.x) stw[t] = twg[(t / V) * (t % V)];
@@ -1508,13 +1515,13 @@ __global__ __launch_bounds__(kBlock) void k_fwd_z(const PoseSlot* __restrict__ s
 // plane write; all threads of the workgroup call it.  TR_IN_PLANE: the
 // transforms' scratch tr lies inside the plane, so every transform waits
 // until no wavefront reads the plane any more.
-template <int N, int PROWS, bool TR_IN_PLANE = false, int NW = 4>
-__device__ __forceinline__ void col_inverse(float2 (&acc)[N / (NW * RegShape<N>::LPW)][RegShape<N>::V], float2* pl,
+template <int N, int PROWS, bool TR_IN_PLANE = false>
+__device__ __forceinline__ void col_inverse(float2 (&acc)[N / (4 * RegShape<N>::LPW)][RegShape<N>::V], float2* pl,
                                             float2* tr, const float2* twr, int lane, int wave, float2* tb, int wx,
                                             int wy, float invG) {
   using RS = RegShape<N>;
   constexpr int L = RS::L, V = RS::V, LPW = RS::LPW;
-  constexpr int LPP = NW * LPW;
+  constexpr int LPP = 4 * LPW;
   constexpr int NPASS = N / LPP;
   // inverse x transforms of the ky lines: value m = x' = n2 + L*m
   int ln = lane % LPW, n2 = lane / LPW;
@@ -3165,7 +3172,7 @@ size_t fwd_reg_lds_bytes(int N, int boxmax, int max_chan_atoms) {
 template <int N>
 constexpr size_t fwd_reg_static() {
   using R = RegShape<N>;
-  return (4 * (size_t)R::SLICE + (R::V >= 16 ? (size_t)R::L * R::V : 1)) * sizeof(float2);
+  return ((size_t)fwd_reg_scratch<N>() + (R::V >= 16 ? (size_t)R::L * R::V : 1)) * sizeof(float2);
 }
 
 namespace {
