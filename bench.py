@@ -306,7 +306,8 @@ def serve_leg(ctx, cdk, workloads, nreq, load, max_batch, seed):
 def fused_steps(cdk, batch, steps, warmup, npose):
     """W untimed and K timed passes of the whole fused search (hipGraph
     replay + result copy-back), each bracketed by device synchronisation
-    inside Batch.run."""
+    inside Batch.run.  A Batch launches its first pass eagerly and captures its
+    graph on the second, so from W = 2 on only replays are timed."""
     for i in range(warmup):
         batch.run(cdk.ENGINE_FUSED)
         log("warmup %d done" % i)
@@ -828,7 +829,7 @@ def main():
     ap = argparse.ArgumentParser(description=__doc__.split("\n")[0])
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=3)
-    ap.add_argument("--warmup", type=int, default=1)
+    ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--workload", choices=["single", "batched", "large"], default="single")
     ap.add_argument("--protein", choices=["p64", "p96", "p128"], default="p64",
                     help="grids of the single-ligand workload (the headline is p64)")
@@ -843,14 +844,14 @@ def main():
     ap.add_argument("--chunk", type=int, default=0, help="poses per fused launch set (0 = from the HBM budget)")
     ap.add_argument("--group", type=int, default=0, help="poses per mid-kernel workgroup (0 = by the launch size)")
     ap.add_argument("--pipeline", type=int, default=-1,
-                    help="fused engine form: 0 planes, 1 columns (64^3), 2 atoms (64^3, 96^3, 128^3), -1 autotuned")
+                    help="fused engine form: 0 planes, 1 columns (64^3), 2 atoms (64^3, 96^3, 128^3), -1 by the context's rule")
     ap.add_argument("--overlap-z", type=int, default=1,
                     help="atom form: overlap each launch set's z-inverse stage with the next set (1) or not (0)")
     ap.add_argument("--atom-products", type=int, default=2,
                     help="atom form products: 2 exact three-part FP16 splits (FP32-accurate), 0 two-part FP16 "
                          "splits, 1 FP32 matrix cores")
-    ap.add_argument("--fwd", type=int, default=-1, help="forward plane form: 0 block, 1 register, -1 autotuned")
-    ap.add_argument("--inv", type=int, default=-1, help="inverse plane form: 0 block, 1 register, -1 autotuned")
+    ap.add_argument("--fwd", type=int, default=-1, help="forward plane form: 0 block, 1 register, -1 by grid edge")
+    ap.add_argument("--inv", type=int, default=-1, help="inverse plane form: 0 block, 1 register, -1 by grid edge")
     ap.add_argument("--serve-requests", type=int, default=40, help="requests in the serving leg (0 = skip)")
     ap.add_argument("--callers", type=int, default=1,
                     help="time the callers either side of the search (retention, rescoring, refinement, grid handoff, conformers)")
