@@ -176,13 +176,13 @@ int cdk_context_set_option(cdk_context* ctx, const char* key, int64_t v) {
               "matrix cores, exact three-part splits)");
       c.atom_products = (int)v;
     } else if (k == "pipeline") {
-      require(v >= -1 && v <= 2, "pipeline must be -1 (tuned), 0 (plane form), 1 (column form) or 2 (atom form)");
+      require(v >= -1 && v <= 2, "pipeline must be -1 (chosen once per grid edge), 0 (plane form), 1 (column form) or 2 (atom form)");
       c.pipeline = (int)v;
     } else if (k == "fwd_variant") {
-      require(v >= -1 && v <= 1, "fwd_variant must be -1 (tuned), 0 (block) or 1 (register)");
+      require(v >= -1 && v <= 1, "fwd_variant must be -1 (by grid edge), 0 (block) or 1 (register)");
       c.fwd_variant = (int)v;
     } else if (k == "inv_variant") {
-      require(v >= -1 && v <= 1, "inv_variant must be -1 (tuned), 0 (block) or 1 (register)");
+      require(v >= -1 && v <= 1, "inv_variant must be -1 (by grid edge), 0 (block) or 1 (register)");
       c.inv_variant = (int)v;
     } else if (k == "use_graph") {
       c.use_graph = v != 0;

@@ -227,7 +227,7 @@ struct Context {
   size_t ws_budget = 8ull << 30;  // bytes of per-batch working arrays
   int ref_batch = 50;             // poses per reference-dataflow batch (NoMini:208)
   int fused_chunk = 0;            // 0 = from budget
-  int mid_group = 0;              // poses per mid-stage workgroup; 0 = tuned
+  int mid_group = 0;              // poses per mid-stage workgroup; 0 = by launch size
   int mid_depth = 0;              // mid-stage register ring depth with a fixed group; 0 = 2
   int mid_poses = 0;              // poses sharing each protein load in the mid stage with a fixed group; 0 = 1
   int pipeline = -1;              // fused pipeline form (kPipePlanes, kPipeColumns, kPipeAtoms); -1 = chosen once per grid edge
