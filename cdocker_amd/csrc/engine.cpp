@@ -996,9 +996,9 @@ namespace {
 
 // t's tables to the device on the context stream (context lock held): through
 // t's pinned staging in one asynchronous copy (one from pageable memory would
-// hold the host until the stream's earlier work is done).  The staging is
-// rewritten only once that copy is over.
-void upload_tables(Context& ctx, Prepared& t) {
+// hold the host until the stream's earlier work is done), the staging rewritten
+// only once that copy is over; or through `scratch` in pieces.
+void upload_tables(Context& ctx, Prepared& t, CallScratch* scratch = nullptr) {
   struct Part {
     DevView* dst;
     const void* src;
@@ -1018,7 +1018,7 @@ void upload_tables(Context& ctx, Prepared& t) {
   const size_t meta = l.add(total * sizeof(RotMeta));
   if (t.h_up_busy) hip_check(hipStreamSynchronize(ctx.stream), "upload sync");
   t.h_up_busy = false;
-  if (tables > t.h_up_cap) {
+  if (!scratch && tables > t.h_up_cap) {
     if (t.h_up) (void)hipHostFree(t.h_up);
     t.h_up = nullptr;
     t.h_up_cap = 0;
@@ -1030,10 +1030,18 @@ void upload_tables(Context& ctx, Prepared& t) {
   char* h = static_cast<char*>(t.h_up);
   for (const Part& p : parts) {
     p.dst->p = d + p.off;
-    if (p.bytes) std::memcpy(h + p.off, p.src, p.bytes);
+    if (!p.bytes) continue;
+    if (scratch) {
+      scratch->in(p.dst->p, p.src, p.bytes);
+      hip_check(hipStreamSynchronize(ctx.stream), "tables H2D");  // the next part reuses the pieces
+    } else {
+      std::memcpy(h + p.off, p.src, p.bytes);
+    }
   }
-  hip_check(hipMemcpyAsync(d, h, tables, hipMemcpyHostToDevice, ctx.stream), "tables H2D");
-  t.h_up_busy = true;
+  if (!scratch) {
+    hip_check(hipMemcpyAsync(d, h, tables, hipMemcpyHostToDevice, ctx.stream), "tables H2D");
+    t.h_up_busy = true;
+  }
   t.d_keys.p = d + keys;
   t.d_meta.p = d + meta;
   t.res_meta = meta - keys;
@@ -1051,9 +1059,7 @@ void prepare_search(Context& ctx, const Protein& prot, const std::vector<Job>& j
 
 namespace {
 
-// Enqueues t's launch sequence and the copies of its keys and per-pose
-// metadata to t's pinned staging;
-// context lock held.
+// Enqueues t's launch sequence (context lock held).
 void enqueue_search(Context& ctx, Prepared& t, Engine engine, bool use_graph, EventTimer& timer,
                     hipEvent_t start = nullptr) {
   const Protein& prot = *t.prot;
@@ -1115,6 +1121,10 @@ void enqueue_search(Context& ctx, Prepared& t, Engine engine, bool use_graph, Ev
       enqueue_fused(ctx, prot, t, chunk, tu, timer);
     }
   }
+}
+
+// Enqueues the copy of t's keys and per-pose metadata to its pinned staging.
+void enqueue_results(Context& ctx, Prepared& t) {
   if (t.res_bytes > t.h_res_cap) {
     if (t.h_res) (void)hipHostFree(t.h_res);
     t.h_res = nullptr;
@@ -1125,14 +1135,10 @@ void enqueue_search(Context& ctx, Prepared& t, Engine engine, bool use_graph, Ev
   hip_check(hipMemcpyAsync(t.h_res, t.d_keys.p, t.res_bytes, hipMemcpyDeviceToHost, ctx.stream), "results D2H");
 }
 
-// Poses first .. first + n - 1 of t from its host staging; index, mincoor, box
-// and win optional ([n][3] each).
-void decode_poses(const Prepared& t, size_t first, size_t n, float* energy, int* index, float* mincoor, int* box,
-                  int* win) {
-  const unsigned long long* keys = static_cast<const unsigned long long*>(t.h_res) + first;
-  const RotMeta* meta =
-      reinterpret_cast<const RotMeta*>(static_cast<const char*>(t.h_res) + t.res_meta) + first;
-  const unsigned N = (unsigned)t.prot->N;
+// n poses' results from their keys and metadata; index, mincoor, box and win
+// optional ([n][3] each).
+void decode_poses(unsigned N, const unsigned long long* keys, const RotMeta* meta, size_t n, float* energy, int* index,
+                  float* mincoor, int* box, int* win) {
   for (size_t i = 0; i < n; ++i) {
     const unsigned long long k = keys[i];
     const RotMeta& m = meta[i];
@@ -1152,6 +1158,12 @@ void decode_poses(const Prepared& t, size_t first, size_t n, float* energy, int*
   }
 }
 
+// t's keys and metadata in its host staging.
+const unsigned long long* staged_keys(const Prepared& t) { return static_cast<const unsigned long long*>(t.h_res); }
+const RotMeta* staged_meta(const Prepared& t) {
+  return reinterpret_cast<const RotMeta*>(static_cast<const char*>(t.h_res) + t.res_meta);
+}
+
 void decode_results(Prepared& t) {
   t.results.assign(t.job_first.size(), PoseResults());
   for (size_t j = 0; j < t.job_first.size(); ++j) {
@@ -1162,7 +1174,9 @@ void decode_results(Prepared& t) {
     r.mincoor.resize(n * 3);
     r.box.resize(n * 3);
     r.win.resize(n * 3);
-    decode_poses(t, t.job_first[j], n, r.energy.data(), r.index.data(), r.mincoor.data(), r.box.data(), r.win.data());
+    const size_t first = t.job_first[j];
+    decode_poses((unsigned)t.prot->N, staged_keys(t) + first, staged_meta(t) + first, n, r.energy.data(),
+                 r.index.data(), r.mincoor.data(), r.box.data(), r.win.data());
   }
 }
 
@@ -1170,9 +1184,45 @@ void decode_results(Prepared& t) {
 void run_prepared(Context& ctx, Prepared& t, Engine engine, bool use_graph) {
   EventTimer timer(ctx);
   enqueue_search(ctx, t, engine, use_graph, timer);
+  enqueue_results(ctx, t);
   hip_check(hipStreamSynchronize(ctx.stream), "search sync");
   t.h_up_busy = false;
   t.ran = true;
+  timer.collect();
+}
+
+// The same with tables too large to keep for the next call: no pinned memory
+// of t's own, its results come through the context's arena in pieces, decoded
+// beside the next piece's copy.
+void run_unstaged(Context& ctx, Prepared& t, Engine engine, CallScratch& scratch, float* energy, int* index,
+                  float* mincoor) {
+  EventTimer timer(ctx);
+  enqueue_search(ctx, t, engine, false, timer);
+  constexpr size_t kPer = kDownPiece / (sizeof(unsigned long long) + sizeof(RotMeta)) & ~(size_t)31, kSlots = 4;
+  constexpr size_t kSlotBytes = kPer * (sizeof(unsigned long long) + sizeof(RotMeta));
+  slot_events(ctx);
+  const size_t total = t.slots.size(), n = (total + kPer - 1) / kPer;
+  char* h = scratch.host(std::min(n, kSlots) * kSlotBytes);
+  auto keys = [&](size_t i) { return reinterpret_cast<unsigned long long*>(h + (i % kSlots) * kSlotBytes); };
+  auto meta = [&](size_t i) { return reinterpret_cast<RotMeta*>(keys(i) + kPer); };
+  auto fetch = [&](size_t i) {
+    const size_t o = i * kPer, len = std::min(kPer, total - o);
+    hip_check(hipMemcpyAsync(keys(i), t.d_keys.as<unsigned long long>() + o, len * sizeof(unsigned long long),
+                             hipMemcpyDeviceToHost, ctx.stream),
+              "keys D2H");
+    hip_check(hipMemcpyAsync(meta(i), t.d_meta.as<RotMeta>() + o, len * sizeof(RotMeta), hipMemcpyDeviceToHost,
+                             ctx.stream),
+              "meta D2H");
+    hip_check(hipEventRecord(ctx.call_events[i % kSlots], ctx.stream), "hipEventRecord");
+  };
+  for (size_t i = 0; i < std::min(n, kSlots); ++i) fetch(i);
+  for (size_t i = 0; i < n; ++i) {
+    const size_t o = i * kPer, len = std::min(kPer, total - o);
+    hip_check(hipEventSynchronize(ctx.call_events[i % kSlots]), "result piece");
+    decode_poses((unsigned)t.prot->N, keys(i), meta(i), len, energy + o, index ? index + o * 3 : nullptr,
+                 mincoor ? mincoor + o * 3 : nullptr, nullptr, nullptr);
+    if (i + kSlots < n) fetch(i + kSlots);
+  }
   timer.collect();
 }
 
@@ -1203,6 +1253,7 @@ void submit_search(Context& ctx, Prepared& t) {
     ctx.time_stages = false;
     try {
       enqueue_search(ctx, t, kEngineFused, false, timer, t.start);
+      enqueue_results(ctx, t);
     } catch (...) {
       ctx.time_stages = ts;
       throw;
@@ -1251,10 +1302,19 @@ void run_search(Context& ctx, const Protein& prot, const Job& job, Engine engine
     build_search(prot, {job}, *t);
     std::lock_guard<std::mutex> lock(ctx.mu);
     hip_check(hipSetDevice(ctx.device), "hipSetDevice");
-    upload_tables(ctx, *t);
-    if (!t->slots.empty()) {
-      run_prepared(ctx, *t, engine, false);
-      decode_poses(*t, 0, t->slots.size(), energy, index, mincoor, nullptr, nullptr);
+    const size_t n = t->slots.size(), most = ctx.scratch_keep / 2;
+    if (n * (sizeof(unsigned long long) + sizeof(RotMeta)) > most) {
+      // not kept for the next call: pinned memory of its own would be made and
+      // freed by each such call (1 000 000 poses at 32^3 260 -> 247 ms)
+      CallScratch scratch(ctx);
+      upload_tables(ctx, *t, &scratch);
+      run_unstaged(ctx, *t, engine, scratch, energy, index, mincoor);
+    } else {
+      upload_tables(ctx, *t);
+      if (n) {
+        run_prepared(ctx, *t, engine, false);
+        decode_poses((unsigned)prot.N, staged_keys(*t), staged_meta(*t), n, energy, index, mincoor, nullptr, nullptr);
+      }
     }
   }
   t->prot = nullptr;

@@ -281,3 +281,30 @@ def test_calls_after_calls_that_failed(ctx):
         assert calls() == want
     lig.close()
     prot.close()
+
+
+@pytest.mark.parametrize("engine", [cdk.ENGINE_FUSED, cdk.ENGINE_REFERENCE])
+def test_searches_too_large_to_keep(ctx, engine):
+    """A search whose tables are not kept for the next call copies them and its
+    results in pieces (one, four slots and more, remainders): bit for bit the
+    results of a kept one, with and without the optional arrays' poses found."""
+    prot = make(ctx, 32, 200)
+    x, q, e, r = cdk.synth_ligand(29, 5)
+    x = np.stack([x, 20.0 * x]).astype(np.float32)  # the second conformer does not fit the grid
+    lig = cdk.Ligand(prot, q, e, r)
+    sizes = (1, 14527, 14528, 14529, 60000) if engine == cdk.ENGINE_FUSED else (70, 15000)
+    try:
+        for n in sizes:
+            say("search not kept, engine %d, 2 x %d poses" % (engine, n))
+            quats = np.resize(cdk.QuaternionUniformSampling(cdk.Rng(n), min(n, 4000)), (n, 4))
+            ctx.set_option("scratch_keep_bytes", 128 << 20)
+            want = cdk.search(ctx, prot, lig, x, quats, engine=engine)
+            ctx.set_option("scratch_keep_bytes", 0)
+            got = cdk.search(ctx, prot, lig, x, quats, engine=engine)
+            assert ctx.get_option("scratch_bytes") == 0
+            assert bits(*got) == bits(*want)
+            assert np.isfinite(want[0][0]).all() and not np.isfinite(want[0][1]).all()
+    finally:
+        ctx.set_option("scratch_keep_bytes", 128 << 20)
+        lig.close()
+        prot.close()
