@@ -23,8 +23,8 @@ as a Poisson stream at a fixed fraction of that capacity; it reports p50/p99
 submit-to-result latency and the served poses/s.
 
 --workload batched runs the uneven-batching workload instead (64 ligands of
-15-60 atoms, 10-100 conformers, 1000 quaternions, one hipGraph-captured launch
-set); --workload large the 128^3 x 9 grids at 0.375 A (50-atom ligand, 50
+15-60 atoms, 10-100 conformers, 1000 quaternions, in one batch);
+--workload large the 128^3 x 9 grids at 0.375 A (50-atom ligand, 50
 conformers x 3000 quaternions, top-10 poses per conformer, 1% of the rotations
 re-scored in FP64 by the oracle).
 """
@@ -693,7 +693,7 @@ def run_single(args, cdk, workloads):
 
 
 def run_batched(args, cdk, workloads):
-    """64 uneven ligands in one hipGraph-captured launch set sequence."""
+    """64 uneven ligands in one launch set sequence (one Batch)."""
     t0 = time.time()
     g = workloads.protein_grids("p64")
     w = workloads.config3()
@@ -734,7 +734,7 @@ def run_batched(args, cdk, workloads):
     confs = [L["conformers"].shape[0] for L in w["ligands"]]
     line(args, "poses scored/sec at 64³×9ch FP32, 64 uneven ligands batched", value, total,
          "uneven batching: 64^3 x 9ch FP32 at 0.5 A, 64 ligands (atoms %d-%d, conformers %d-%d) x 1000 "
-         "quaternions = %d poses in one hipGraph" % (min(atoms), max(atoms), min(confs), max(confs), npose),
+         "quaternions = %d poses in one batch" % (min(atoms), max(atoms), min(confs), max(confs), npose),
          {"grid_edge": N, "ligands": len(ligs), "poses": npose, "valid_poses": n_valid,
           "engine": "fused" + ("" if args.no_graph else "+hipGraph")},
          roof, kernels, cpu, reference_engine=ref, per_ligand_identical_first4=same)

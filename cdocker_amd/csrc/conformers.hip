@@ -64,9 +64,9 @@ __device__ __forceinline__ double dot(double ax, double ay, double az, double bx
 // global load: the turn by theta - phi comes from the angle sums, with cos phi
 // and sin phi the dihedral's two components over their length.  Which atoms a
 // rotor moves, and which partners the clash test of an atom skips, are bits in
-// one 64-bit word per atom.  Measured, trials of a 40-atom chain: 565 us for
-// 20 000 (with atan2, cos and sin per rotor, and byte masks) -> 86 us for the
-// 4 096 of a first set.  The components' rounding would stretch the turned
+// one 64-bit word per atom.  Measured, 20 000 trials of a 40-atom chain: 575 us
+// with atan2, cos and sin per rotor and byte masks -> 353 us; a first set of
+// 4 096 takes 86 us.  The components' rounding would stretch the turned
 // atoms a little with every rotor, so the turn is brought to unit length and
 // sums of products are fused.  Error against quadruple precision over 2 000
 // trials of 40-atom chains, r.m.s. / mean largest of a chain, in A: 4.2e-14 /

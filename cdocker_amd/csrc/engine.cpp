@@ -235,8 +235,8 @@ void protein_setup(Protein& p, int nch, int N, float h, const float* mid, const 
 }
 
 // Forward R2C of every channel (NoMini:177-199) plus the copies the fused
-// mid stages read (line-blocked; kz-plane and matrix-core blocks at grid
-// edge 64).
+// mid stages read (line-blocked; kz-plane blocks at grid edge 64, matrix-core
+// blocks at 64, 96 and 128).
 void protein_spectra(Protein& p) {
   Context& ctx = *p.ctx;
   hip_check(launch_r2c_3d(ctx.stream, p.N, p.grid.as<float>(), p.spec.as<float2>(), p.nch, ctx.twiddle(p.N)),

@@ -25,18 +25,13 @@
 namespace cdk {
 
 // ---------------------------------------------------------------------------
-// Plans per grid edge.  The tuned radix list is selected at run time among
-// the variants compiled here (see tune_*).
+// Plans per grid edge.
 // ---------------------------------------------------------------------------
 using P32a = Plan<32, 8, 4>;
 using P48a = Plan<48, 16, 3>;
-using P48b = Plan<48, 4, 4, 3>;
 using P64a = Plan<64, 8, 8>;
-using P64b = Plan<64, 4, 4, 4>;
 using P96a = Plan<96, 8, 4, 3>;
-using P96b = Plan<96, 16, 2, 3>;
 using P128a = Plan<128, 8, 16>;
-using P128b = Plan<128, 4, 4, 8>;
 
 // ---------------------------------------------------------------------------
 // Ordered 64-bit argmin key: high word = float bits mapped to unsigned order,
@@ -839,7 +834,7 @@ __global__ __launch_bounds__(kBlock) void k_fwd_planes_reg(const PoseSlot* __res
 // global memory already in the register layout the transform wants, and the
 // forward output layout is the inverse's input layout.  A workgroup is 4
 // wavefronts and walks a group of poses as one sequence of (pose, channel)
-// items; a ring of DEPTH register buffers (DEPTH tuned, 1 for long lines)
+// items; a ring of DEPTH register buffers (2 or 3, 1 for long lines)
 // keeps the next items' loads in flight while one item is transformed.  When the
 // pose's box is at most N/2 the upper half of every line is zero: those rows
 // are not loaded and the first DFT stage is pruned.  Workgroups map to
@@ -2318,9 +2313,14 @@ struct AtomTab {
 // at two wavefronts per SIMD and up to 256 registers.  A workgroup takes the
 // planes 2 i and 2 i + 1 of a group of poses.
 //
-// What bounds it: a step of 8 entries is 24 matrix-core instructions (768
-// cycles) beside ~106 vector instructions, and the two overlap only as far as
-// the wavefronts' instruction streams are interleaved.  Four wavefronts per
+// What bounds it: vector issue (0.60 of the SIMD cycles) beside the matrix
+// cores (0.31); the two overlap only as far as the wavefronts' instruction
+// streams are interleaved.  A pose of 40 atoms and nine channels takes a
+// wavefront ~5 100 vector and 332 matrix-core instructions (counted): 14 steps
+// of 8 entries, each 24 matrix-core instructions (768 cycles) beside 110
+// vector ones, make 1 500 of them, the nine channel ends of ~146 1 300, the
+// inverse transforms and the store 1 250, the y table, the entries and the
+// first operands the rest.  Four wavefronts per
 // plane at four per SIMD (k_mid_atoms) built every operand twice (141 vector
 // instructions per block and step, most of the splits at half rate), waited
 // on one table lookup after the other, and on each protein load in turn.
@@ -2672,12 +2672,15 @@ __global__ __launch_bounds__(128 * AtomTab::NP) __attribute__((amdgpu_waves_per_
 // y rows only.  Bound by latency: how many wavefronts the tile's LDS and the
 // registers let run.  So the transforms trade values between lanes
 // (lane_fft), with no LDS and no barrier, and the tile holds x' in two turns.
-// Alone per search, with the whole tile overlaying the transforms' LDS
-// scratch (two of three wavefronts transforming at a time at 96) before: 96
-// (2,000 poses) 2.34 -> 2.31 ms, 128 (1,000) 2.41 -> 2.03; the small tile
-// also fits beside the forward kernel's workgroups: the overlapped searches
-// 9.2 -> 8.8 and 10.8 -> 10.45 ms.  The whole tile with lane_fft: 2.00 / 2.44
-// alone, 9.2 / 11.1 overlapped.
+// Alone per search (both builds in one process, calls in turn), with the whole
+// tile overlaying the transforms' LDS scratch (two of three wavefronts
+// transforming at a time at 96) before: 128 (1,000 poses of 40 atoms) 2.63 ->
+// 2.22 ms; 96 (2,000) 2.59 -> 2.65, but the small tile fits beside the forward
+// kernel's workgroups: the overlapped searches, kernels and call, 9.90 -> 9.70
+// ms at 96, 12.06 -> 11.62 at 128 (50 atoms).  At 96 the kernel needs 136
+// registers and is held to 128, 7 of them spilled (0.27 MB written per pose):
+// three wavefronts per SIMD without the spill take the same time alone and 1%
+// more overlapped.
 template <>
 __device__ __forceinline__ unsigned atom_tw_bytes<96>(unsigned k, unsigned i) {
   const unsigned t = mul_u24(k, i);

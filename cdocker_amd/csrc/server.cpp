@@ -12,9 +12,9 @@ void Batch::run(Engine engine) {
     prepare();
   }
   // Capturing and instantiating the graph costs more than the launches it
-  // replaces (16 ligands, 8 launch sets: ~1 ms beside a 6.6 ms run), so a
-  // batch run once is launched eagerly and the graph is made when it runs
-  // again.
+  // replaces (3 ligands: 40 us with one launch set, 180 with four, 0.4 ms with
+  // twenty-four), so a batch run once is launched eagerly and the graph is made
+  // when it runs again.
   execute_search(*ctx, prep, engine, ctx->use_graph && prep.ran);
 }
 
